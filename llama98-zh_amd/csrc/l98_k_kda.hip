@@ -488,11 +488,11 @@ __global__ __launch_bounds__(4 * KD) void k_kda_items(KdaStepArgs b, const KdaIt
 //                the gate rows, the l2 norms, beta and k.q, i.e. everything
 //                that does not read the state, stored as one record per
 //                (row, head): [kn.g | qn.g*scale... | g | kn | v | beta, k.q];
-//   k_kda_rec  - one block per head: the token-serial recurrence over all n
-//                rows from the records, staged through LDS one block of rows
-//                ahead (the next block's records are in flight while the
-//                current block's tokens run); o to orow, the final state to
-//                the base slot;
+//   k_kda_rec  - one block per head and group of state columns: the
+//                token-serial recurrence over all n rows from the records,
+//                staged through LDS one block of rows ahead (the next block's
+//                records are in flight while the current block's tokens run);
+//                o to orow, the final state to the base slot;
 //   k_kda_post - every (row block, head) at once: the gated norm and the
 //                quantization for o_proj, and the conv history after the last
 //                row into the base slot (after every read of it).
@@ -512,77 +512,252 @@ __global__ __launch_bounds__(4 * KD) void k_kda_pre(KdaStepArgs b, int n) {
     kda_step_body<KD, K, MAX_CHUNK, true>(a, blockIdx.y);
 }
 
-// A stage of k_kda_rec: the records of rows s0 .. s0 + MAX_CHUNK - 1 (those
-// below n) of one head, RS4 float4 each, spread over the block's threads
-// (three float4 per thread for every kd here; indices past the stage clamp
-// to its last float4); fetched into registers, later stored to the stage's
-// LDS buffer.
+// k_kda_rec's split.  The state's columns are independent, and a column's u
+// = S^T(g.k) and w = S^T(g.q) are two serial chains of kd adds, of which
+// only u feeds the next state.  A wave issues one VALU instruction per 4
+// cycles, a dependent add included (two waves of a SIMD overlap fully), so
+// the time per token is the instruction count of the wave that carries u:
+//   * a column's state is spread over REC_P = kd / 8 lanes (8 rows each), so
+//     products and state update cost 8 lanes' worth of work while the chain
+//     walks over the lanes (DPP shift by one lane, 8 adds per lane);
+//   * two waves of a block carry u (and delta, left in LDS), two others carry
+//     w and o over the previous stage's tokens with their own copy of the
+//     state, updated from the same delta with the same operations; the w
+//     waves also load the next stage, and leave o in LDS for the u waves to
+//     store a stage later (a wave that both loads and stores would wait for
+//     its stores with its loads, at every stage);
+//   * a block holds 128 / REC_P columns; the grid is (heads, column blocks),
+//     so that a head's blocks share an XCD (heads a multiple of 8) and its
+//     records are read into one L2.
+// One block of 4 kd threads per head with both chains in every wave took
+// 0.63 us (kd = 64) and 1.5 us (kd = 128) per token: about 245 and 470
+// instructions per token on one or two waves per SIMD of 16 CUs.  This split
+// measures 0.29 and 0.44 us (511 rows of 16 heads, alone on the card), about
+// 125 and 200 instructions; the chain alone is 0.11 and 0.21 us.  Stages of 16
+// tokens measured 3 % faster for twice the LDS, which other streams' blocks
+// need.
+#define REC_THREADS 256
 template <int KD>
-struct RecStage {
-    static constexpr int RS4 = (5 * KD + 4) / 4, NTHR = 4 * KD;
-    static_assert(MAX_CHUNK * RS4 <= 3 * NTHR && MAX_CHUNK * RS4 > 2 * NTHR, "three float4 per thread");
-    float4 v0, v1, v2;
-    __device__ __forceinline__ int idx(int u, int m) const { return imin(u * NTHR + (int)threadIdx.x, m - 1); }
-    __device__ __forceinline__ float4 ld(const float *src, size_t rstride, int s0, int f) const {
-        const int t = f / RS4;
-        return reinterpret_cast<const float4 *>(src + (size_t)(s0 + t) * rstride)[f - t * RS4];
-    }
-    __device__ __forceinline__ void fetch(const float *src, size_t rstride, int s0, int n) {
-        const int m = imin(MAX_CHUNK, n - s0) * RS4;
-        v0 = ld(src, rstride, s0, idx(0, m));
-        v1 = ld(src, rstride, s0, idx(1, m));
-        v2 = ld(src, rstride, s0, idx(2, m));
-    }
-    __device__ __forceinline__ void put(float (*buf)[5 * KD + 4], int s0, int n) const {
-        const int m = imin(MAX_CHUNK, n - s0) * RS4;
-        const int f0 = idx(0, m), f1 = idx(1, m), f2 = idx(2, m);      // clamped lanes rewrite the last value
-        reinterpret_cast<float4 *>(buf[f0 / RS4])[f0 % RS4] = v0;
-        reinterpret_cast<float4 *>(buf[f1 / RS4])[f1 % RS4] = v1;
-        reinterpret_cast<float4 *>(buf[f2 / RS4])[f2 % RS4] = v2;
-    }
+struct Rec {
+    static constexpr int P = KD / 8, CPB = 128 / P, T = MAX_CHUNK;
+    static constexpr int F4 = KD + CPB / 4 + 1;         // float4 of a staged row: c, a, g, b, own v, beta / kq
+    static constexpr int RSL = 4 * F4;                  // its floats
+    static constexpr int NL = (T * F4 + 127) / 128;     // per thread of the w waves, which stage them
+    static_assert(P == 4 || P == 8 || P == 16, "a column within a 16-lane row");
+    static_assert(KD % CPB == 0 && CPB % 4 == 0, "whole column blocks");
 };
 
-template <int KD>
-__global__ __launch_bounds__(4 * KD) void k_kda_rec(KdaStepArgs a, int n) {
-    constexpr int RPL = KD / 4, RS = 5 * KD + 4, T = MAX_CHUNK;
-    __shared__ __align__(16) float s_rec[2][T][RS];
-    const int h = blockIdx.x, tid = threadIdx.x, col = tid >> 2, row0 = (tid & 3) * RPL;
-    float4 *sp = reinterpret_cast<float4 *>(a.state + (size_t)(*a.ctl_slot) * a.slot_stride + (size_t)h * KD * KD) + tid;
-    float S[RPL];
+// A lane's rows of one token: x = kn.g (u) or qn.g*scale (w), g, b = kn; s0, s1
+// v and beta (u) or delta and k.q (w).
+struct RecTok {
+    v4f x0, x1, g0, g1, b0, b1;
+    float s0, s1;
+};
+
+// The chain over a column's lanes: lane 0 sums its products from 0 in order,
+// lane 1 continues from lane 0's sum, ...; the last lane of the column ends
+// with the whole sum (the others with partial sums nobody reads).
+template <int P>
+__device__ __forceinline__ float rec_chain(const float (&p)[8]) {
+    float u = 0.0f;
 #pragma unroll
-    for (int i = 0; i < RPL / 4; i++) {
-        const float4 q = sp[i * 4 * KD];
-        S[4 * i] = q.x; S[4 * i + 1] = q.y; S[4 * i + 2] = q.z; S[4 * i + 3] = q.w;
+    for (int i = 0; i < 8; i++) u += p[i];
+#pragma unroll
+    for (int ph = 1; ph < P; ph++) {
+        // row_shr:1
+        u = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(u), 0x111, 0xF, 0xF, true)) + p[0];
+#pragma unroll
+        for (int i = 1; i < 8; i++) u += p[i];
     }
-    const size_t rstride = (size_t)a.nv * RS;
-    const float *src = a.rec + (size_t)h * RS;
-    RecStage<KD> nb;
-    nb.fetch(src, rstride, 0, n);
-    nb.put(s_rec[0], 0, n);
+    return u;
+}
+// Every lane of a column <- its last lane.
+template <int P>
+__device__ __forceinline__ float rec_bcast(float v) {
+    const int x = __float_as_int(v);
+    if constexpr (P == 16) return __int_as_float(__builtin_amdgcn_update_dpp(0, x, 0x15F, 0xF, 0xF, true));  // row_newbcast:15
+    const int q = __builtin_amdgcn_update_dpp(0, x, 0xFF, 0xF, 0xF, true);                    // quad_perm [3,3,3,3]
+    if constexpr (P == 4) return __int_as_float(q);
+    // the lower quad of each 8 lanes takes the upper one's (row_half_mirror, banks 0 and 2)
+    return __int_as_float(__builtin_amdgcn_update_dpp(q, q, 0x141, 0xF, 0x5, false));
+}
+__device__ __forceinline__ void rec_products(float (&p)[8], const float (&S)[8], const RecTok &k) {
+    p[0] = S[0] * k.x0.x; p[1] = S[1] * k.x0.y; p[2] = S[2] * k.x0.z; p[3] = S[3] * k.x0.w;
+    p[4] = S[4] * k.x1.x; p[5] = S[5] * k.x1.y; p[6] = S[6] * k.x1.z; p[7] = S[7] * k.x1.w;
+}
+__device__ __forceinline__ void rec_decay(float (&d)[8], const float (&S)[8], const RecTok &k) {
+    d[0] = S[0] * k.g0.x; d[1] = S[1] * k.g0.y; d[2] = S[2] * k.g0.z; d[3] = S[3] * k.g0.w;
+    d[4] = S[4] * k.g1.x; d[5] = S[5] * k.g1.y; d[6] = S[6] * k.g1.z; d[7] = S[7] * k.g1.w;
+}
+__device__ __forceinline__ void rec_update(float (&S)[8], const float (&d)[8], const RecTok &k, float ut) {
+    S[0] = d[0] + k.b0.x * ut; S[1] = d[1] + k.b0.y * ut; S[2] = d[2] + k.b0.z * ut; S[3] = d[3] + k.b0.w * ut;
+    S[4] = d[4] + k.b1.x * ut; S[5] = d[5] + k.b1.y * ut; S[6] = d[6] + k.b1.z * ut; S[7] = d[7] + k.b1.w * ut;
+}
+
+// A stage's nt tokens.  A whole stage is straight-line code (no loop or
+// address arithmetic on the waves that set the pace, exact LDS waits), the
+// next token's rows arriving during the current one.
+template <int T, class Load, class Step>
+__device__ __forceinline__ void rec_tokens(int nt, Load &&load, Step &&step) {
+    RecTok A, B;
+    if (nt == T) {
+        load(A, 0);
+#pragma unroll
+        for (int t = 0; t < T; t += 2) {
+            load(B, t + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            step(A, t);
+            if (t + 2 < T) load(A, t + 2);
+            __builtin_amdgcn_sched_barrier(0);
+            step(B, t + 1);
+        }
+        return;
+    }
+#pragma unroll 1
+    for (int t = 0; t < nt; t++) {
+        load(A, t);
+        step(A, t);
+    }
+}
+
+template <int KD>
+__global__ __launch_bounds__(REC_THREADS) void k_kda_rec(KdaStepArgs a, int n) {
+    using R = Rec<KD>;
+    constexpr int P = R::P, CPB = R::CPB, T = R::T, F4 = R::F4, RSL = R::RSL, NL = R::NL, RS = 5 * KD + 4;
+    // stage sk is read by the u waves while the w waves read stage sk - 1 and
+    // stage sk + 1 arrives; stage sk - 2's outputs leave
+    __shared__ __align__(16) float s_rec[3][T][RSL];
+    __shared__ float s_ut[2][T][CPB], s_o[2][T * CPB];
+    const int h = blockIdx.x, tid = threadIdx.x, l = tid & 127;
+    const bool uw = tid < 128;                            // (uniform per wave)
+    const int cl = l / P, p = l - cl * P, col = blockIdx.y * CPB + cl, row0 = 8 * p;
+    // the ring slot's float4 of rows 4 m .. 4 m + 3 (m = 2 p, 2 p + 1) of the column
+    float4 *st = reinterpret_cast<float4 *>(a.state + (size_t)(*a.ctl_slot) * a.slot_stride + (size_t)h * KD * KD);
+    auto slot4 = [&](int m) { return (m % (KD / 16)) * 4 * KD + 4 * col + m / (KD / 16); };
+    float S[8];
+    {
+        const float4 q0 = st[slot4(2 * p)], q1 = st[slot4(2 * p + 1)];
+        S[0] = q0.x; S[1] = q0.y; S[2] = q0.z; S[3] = q0.w;
+        S[4] = q1.x; S[5] = q1.y; S[6] = q1.z; S[7] = q1.w;
+    }
+    // staged float4 f of a thread: row f / F4, the block's part of its record
+    const v4f *src = reinterpret_cast<const v4f *>(a.rec + (size_t)h * RS);
+    const int rstride4 = a.nv * (RS / 4);
+    int srow[NL], soff[NL];
+#pragma unroll
+    for (int u = 0; u < NL; u++) {
+        const int f = imin(u * 128 + l, T * F4 - 1), t = f / F4, e = f - t * F4;
+        srow[u] = t;
+        soff[u] = e < KD ? e : e < KD + CPB / 4 ? e + (int)blockIdx.y * (CPB / 4) : 5 * (KD / 4);
+    }
+    v4f nb[NL];
+    auto fetch = [&](int s0) {                            // rows past the last repeat it
+#pragma unroll
+        for (int u = 0; u < NL; u++) nb[u] = src[(size_t)imin(s0 + srow[u], n - 1) * rstride4 + soff[u]];
+    };
+    auto put = [&](int b) {
+#pragma unroll
+        for (int u = 0; u < NL; u++)
+            reinterpret_cast<v4f *>(&s_rec[b][0][0])[imin(u * 128 + l, T * F4 - 1)] = nb[u];
+    };
+    if (!uw) {
+        fetch(0);
+        put(0);
+    }
+    // the state's loads retired here: pending at the loop, the compiler would
+    // wait at every stage's start for all loads, the next stage's among them
+#pragma unroll
+    for (int i = 0; i < 8; i++) asm volatile("" : "+v"(S[i]));
     __syncthreads();
     const int nst = (n + T - 1) / T;
+    int bu = 0, bw = 2;                                   // buffers of stages sk and sk - 1
 #pragma unroll 1
-    for (int sk = 0; sk < nst; sk++) {
-        // the next stage's records are in flight while this stage runs (the
-        // last stage refetches itself into the idle buffer)
-        const int sb = sk & 1, s0 = sk * T, nt = imin(T, n - s0), sn = sk + 1 < nst ? s0 + T : s0;
-        nb.fetch(src, rstride, sn, n);
-#pragma unroll 1
-        for (int t = 0; t < nt; t++) {
-            const float *rc = s_rec[sb][t];
-            const float o = kda_token<KD>(S, rc, rc + KD, rc + 2 * KD, rc + 3 * KD, rc + 4 * KD + col, rc + 5 * KD,
-                                          rc + 5 * KD + 1, row0);
-            if ((tid & 3) == 0) {
-                const size_t oi = (size_t)(s0 + t) * a.value + (size_t)h * KD + col;
-                a.orow[oi] = o;
-                if (a.raw_out) a.raw_out[oi] = o;
-            }
-        }
-        nb.put(s_rec[sb ^ 1], sn, n);
-        __syncthreads();
-    }
+    for (int sk = 0; sk < nst + 2; sk++) {
+        const int bn = bu == 2 ? 0 : bu + 1;              // stage sk + 1's (last read as stage sk - 2)
+        if (uw) {
+            // stage sk - 2's outputs: read now, stored after this stage's tokens
+            constexpr int NO = (T * CPB + 127) / 128;
+            float ov[NO];
 #pragma unroll
-    for (int i = 0; i < RPL / 4; i++) sp[i * 4 * KD] = make_float4(S[4 * i], S[4 * i + 1], S[4 * i + 2], S[4 * i + 3]);
+            for (int i = 0; i < NO; i++) ov[i] = s_o[sk & 1][imin(128 * i + l, T * CPB - 1)];
+            if (sk < nst) {
+                const int nt = imin(T, n - sk * T);
+                const float(*rec)[RSL] = s_rec[bu];
+                float *ut_out = &s_ut[sk & 1][0][cl];
+                auto load = [&](RecTok &k, int t) {
+                    const float *rc = rec[t];
+                    k.x0 = *reinterpret_cast<const v4f *>(&rc[row0]);
+                    k.x1 = *reinterpret_cast<const v4f *>(&rc[row0 + 4]);
+                    k.s0 = rc[4 * KD + cl];
+                    k.s1 = rc[4 * KD + CPB];
+                    k.g0 = *reinterpret_cast<const v4f *>(&rc[2 * KD + row0]);
+                    k.g1 = *reinterpret_cast<const v4f *>(&rc[2 * KD + row0 + 4]);
+                    k.b0 = *reinterpret_cast<const v4f *>(&rc[3 * KD + row0]);
+                    k.b1 = *reinterpret_cast<const v4f *>(&rc[3 * KD + row0 + 4]);
+                };
+                auto step = [&](const RecTok &k, int t) {
+                    float pr[8], d[8];
+                    rec_products(pr, S, k);
+                    rec_decay(d, S, k);
+                    const float u = rec_bcast<P>(rec_chain<P>(pr));
+                    const float ut = (k.s0 - 1.0f * u) * k.s1;
+                    rec_update(S, d, k, ut);
+                    if (p == 0) ut_out[t * CPB] = ut;
+                };
+                rec_tokens<T>(nt, load, step);
+            }
+            if (sk > 1) {
+                const int s0 = (sk - 2) * T, nt = imin(T, n - s0);
+#pragma unroll
+                for (int i = 0; i < NO; i++) {
+                    const int f = 128 * i + l, t = f / CPB;
+                    if (t < nt) {
+                        const size_t oi = (size_t)(s0 + t) * a.value + (size_t)h * KD + blockIdx.y * CPB + f - t * CPB;
+                        a.orow[oi] = ov[i];
+                        if (a.raw_out) a.raw_out[oi] = ov[i];
+                    }
+                }
+            }
+        } else {
+            fetch(imin(sk + 1, nst - 1) * T);
+            __builtin_amdgcn_sched_barrier(0);
+            if (sk > 0 && sk <= nst) {
+                const int nt = imin(T, n - (sk - 1) * T);
+                const float(*rec)[RSL] = s_rec[bw];
+                const float *ut_in = &s_ut[(sk - 1) & 1][0][cl];
+                float *o_out = &s_o[(sk - 1) & 1][cl];
+                auto load = [&](RecTok &k, int t) {
+                    const float *rc = rec[t];
+                    k.x0 = *reinterpret_cast<const v4f *>(&rc[KD + row0]);
+                    k.x1 = *reinterpret_cast<const v4f *>(&rc[KD + row0 + 4]);
+                    k.s0 = ut_in[t * CPB];
+                    k.s1 = rc[4 * KD + CPB + 1];
+                    k.g0 = *reinterpret_cast<const v4f *>(&rc[2 * KD + row0]);
+                    k.g1 = *reinterpret_cast<const v4f *>(&rc[2 * KD + row0 + 4]);
+                    k.b0 = *reinterpret_cast<const v4f *>(&rc[3 * KD + row0]);
+                    k.b1 = *reinterpret_cast<const v4f *>(&rc[3 * KD + row0 + 4]);
+                };
+                auto step = [&](const RecTok &k, int t) {
+                    float pr[8], d[8];
+                    rec_products(pr, S, k);
+                    rec_decay(d, S, k);
+                    const float w = rec_chain<P>(pr);
+                    rec_update(S, d, k, k.s0);
+                    const float o = 1.0f * w + k.s0 * k.s1;
+                    if (p == P - 1) o_out[t * CPB] = o;
+                };
+                rec_tokens<T>(nt, load, step);
+            }
+            put(bn);
+        }
+        __syncthreads();
+        bw = bu;
+        bu = bn;
+    }
+    if (uw) {
+        st[slot4(2 * p)] = make_float4(S[0], S[1], S[2], S[3]);
+        st[slot4(2 * p + 1)] = make_float4(S[4], S[5], S[6], S[7]);
+    }
 }
 
 template <int KD, int K>
@@ -703,7 +878,7 @@ extern "C" int l98k_kda_split(const KdaStepArgs *a, int n, int kd, int K, hipStr
 #define KDA_SPLIT(KD_, K_)                                                                            \
     do {                                                                                              \
         hipLaunchKernelGGL((k_kda_pre<KD_, K_>), rows, dim3(4 * (KD_)), 0, st, *a, n);               \
-        hipLaunchKernelGGL((k_kda_rec<KD_>), dim3(a->nv), dim3(4 * (KD_)), 0, st, *a, n);            \
+        hipLaunchKernelGGL((k_kda_rec<KD_>), dim3(a->nv, (KD_) / Rec<KD_>::CPB), dim3(REC_THREADS), 0, st, *a, n); \
         hipLaunchKernelGGL((k_kda_post<KD_, K_>), rows, dim3(4 * (KD_)), 0, st, *a, n);              \
     } while (0)
     switch (kd * 8 + K) {
