@@ -18,13 +18,10 @@
 // bytes each, and receives D[4 (l / 16) + v][l % 16] in result register v.
 // A is the weight tile (rows), B the activation tile (tokens).
 //
-// A block computes MF_ROWS = 16 MF_RT weight rows x 64 token columns (a
-// wave per 16 columns, MF_RT 16-row MFMA tiles each; two tiles keep a
-// wave's per-group fp32 fold short and give a 1024-row GEMM a block per CU).  K goes through LDS in stages of MF_KC bytes (eight groups),
-// double-buffered: each thread loads its 16-byte pieces of the next stage
-// (coalesced: 16 threads per 256-byte row) while the block's MFMAs run on
-// the current one, so a stage costs one memory round trip overlapped with
-// compute instead of one per group batch.
+// Two kernels: k_mfma_q8t for K a multiple of 128 (every configuration of
+// bench.py), and k_mfma_q8 for any K (the toy models' 32, 64, 96, ...): blocks
+// of 16 weight rows x 64 token columns (a wave per 16 columns), K through
+// double-buffered LDS stages of MF_KC bytes (eight groups).
 #include "l98_devmath.h"
 
 typedef int v4i_t __attribute__((ext_vector_type(4)));
@@ -109,14 +106,13 @@ __device__ __forceinline__ void mf_fold(float (&f)[4], v4i_t d, float s, bool on
     f[2] += one ? (float)d[2] : (float)d[2] * s;
     f[3] += one ? (float)d[3] : (float)d[3] * s;
 }
-template <bool FULL>
 __device__ __forceinline__ void mf_stage(float (&f)[MF_RT][4], const int8_t (*sw)[MF_LDS_ROW],
                                          const int8_t (*sx)[MF_LDS_ROW], const float *sc, int ng, bool one,
                                          int wave, int lane, int kq) {
     const v4i_t zero = {0, 0, 0, 0};
 #pragma unroll
     for (int gl = 0; gl < MF_KC / 32; gl++) {
-        if (!FULL && gl >= ng) break;                  // uniform
+        if (gl >= ng) break;                           // uniform
         const long b = *reinterpret_cast<const long *>(&sx[16 * wave + (lane & 15)][32 * gl + kq]);
         const long a0 = *reinterpret_cast<const long *>(&sw[(lane & 15)][32 * gl + kq]);
         const v4i_t d0 = __builtin_amdgcn_mfma_i32_16x16x32_i8(a0, b, zero, 0, 0, 0);
@@ -143,7 +139,6 @@ __device__ __forceinline__ void mf_stage(float (&f)[MF_RT][4], const int8_t (*sw
     }
 }
 
-template <bool FULLK>
 __global__ __launch_bounds__(MF_THREADS) void k_mfma_q8(const int8_t *__restrict__ W0, const float *__restrict__ ws0,
                                                          int N0, int K0, size_t w_group_stride,
                                                          const int8_t *__restrict__ X0, const float *__restrict__ Xs0,
@@ -251,18 +246,11 @@ __global__ __launch_bounds__(MF_THREADS) void k_mfma_q8(const int8_t *__restrict
             const float *sc = s_xs[buf][16 * wave + (lane & 15)];
             // the next stage's loads are in flight during this stage's MFMAs (the
             // last stage reloads itself into the idle buffer); the scheduling
-            // barrier keeps their issue ahead of the MFMAs.  FULLK: every stage
-            // holds eight groups and the stage is one basic block (with a
-            // branch between them the compiler sinks the loads to their LDS
-            // stores).
+            // barrier keeps their issue ahead of the MFMAs
             MF_STAGE_LOAD(A, st + 1 < nst ? st + 1 : st);
             __builtin_amdgcn_sched_barrier(0);
-            if constexpr (FULLK) {
-                mf_stage<true>(f, s_w[buf], s_x[buf], sc, MF_KC / 32, false, wave, lane, kq);
-            } else {
-                mf_stage<false>(f, s_w[buf], s_x[buf], sc, nb - st * (MF_KC / 32), one, wave, lane, kq);
-                if (one) s0 = sc[0];
-            }
+            mf_stage(f, s_w[buf], s_x[buf], sc, nb - st * (MF_KC / 32), one, wave, lane, kq);
+            if (one) s0 = sc[0];
             MF_STAGE_PUT(A, buf ^ 1);
             __syncthreads();
         }
@@ -290,76 +278,71 @@ __global__ __launch_bounds__(MF_THREADS) void k_mfma_q8(const int8_t *__restrict
 #undef MF_STAGE_LOAD
 #undef MF_STAGE_PUT
 
-// The narrow form: a block computes 64 weight rows x 16 token columns
-// (wave w: rows 16 w .. 16 w + 15 of the same 16 columns), so each block
-// streams four times the weights of k_mfma_q8's 16-row tile and stages
-// only the 16 columns it uses, and the loads run two stages ahead (register
-// sets A and B alternate) - for few columns per weight tile (the experts of
-// a batched verify, whose groups average a few pairs; dense GEMMs over the
-// batch's rows), where a stage's round trip, not the arithmetic, bounds the
-// block.  Dense (cols.list null: column t is activation and output row t,
-// t < M; jobs as in k_mfma_q8; a 1-D grid mapped onto the XCDs so that the
-// column tiles of a weight tile share an L2) or grouped (block z is group g; a group's
-// column tiles spread over the grid's y, whose extra blocks exit at once).
-// Same stages, MFMAs and fold per (row, column) as k_mfma_q8, so the same
-// bits.
-#define MFN_ROWS 64
-#define MFN_COLS 16
-#define MFN_DENSE_MAX 128      // dense GEMMs of at most this many rows take the narrow tiles
-#define MFN_STAGE_LOAD(R, st_)                                                                 \
-    do {                                                                                       \
-        const int off_ = imin((st_) * MF_KC + 16 * pc, K - 16);                                \
-        R##w0 = *reinterpret_cast<const int4 *>(wl0 + off_);                                   \
-        R##w1 = *reinterpret_cast<const int4 *>(wl1 + off_);                                   \
-        R##w2 = *reinterpret_cast<const int4 *>(wl2 + off_);                                   \
-        R##w3 = *reinterpret_cast<const int4 *>(wl3 + off_);                                   \
-        R##x0 = *reinterpret_cast<const int4 *>(xl0 + off_);                                   \
-        if (tid < 64) {                                                                        \
-            const int g_ = (st_) * (MF_KC / 32) + 2 * (tid & 3);                               \
-            R##t0 = xsl[imin(g_, nb - 1)];                                                     \
-            R##t1 = xsl[imin(g_ + 1, nb - 1)];                                                 \
-        }                                                                                      \
-    } while (0)
-#define MFN_STAGE_PUT(R, b_)                                                                   \
-    do {                                                                                       \
-        *reinterpret_cast<int4 *>(&s_w[b_][rr][16 * pc]) = R##w0;                              \
-        *reinterpret_cast<int4 *>(&s_w[b_][rr + 16][16 * pc]) = R##w1;                         \
-        *reinterpret_cast<int4 *>(&s_w[b_][rr + 32][16 * pc]) = R##w2;                         \
-        *reinterpret_cast<int4 *>(&s_w[b_][rr + 48][16 * pc]) = R##w3;                         \
-        *reinterpret_cast<int4 *>(&s_x[b_][rr][16 * pc]) = R##x0;                              \
-        if (tid < 64) *reinterpret_cast<float2 *>(&s_xs[b_][tid >> 2][2 * (tid & 3)]) = make_float2(R##t0, R##t1); \
-    } while (0)
-template <bool FULLK>
-__global__ __launch_bounds__(MF_THREADS) void k_mfma_q8n(const int8_t *__restrict__ W0, const float *__restrict__ ws0,
-                                                          int N0, int K0, size_t w_group_stride,
-                                                          const int8_t *__restrict__ X0, const float *__restrict__ Xs0,
-                                                          int M, MfCols cols, float *__restrict__ out0,
-                                                          int out_stride0, MfJobs jobs) {
-    __shared__ __align__(16) int8_t s_w[2][MFN_ROWS][MF_LDS_ROW];
-    __shared__ __align__(16) int8_t s_x[2][MFN_COLS][MF_LDS_ROW];
-    __shared__ __align__(16) float s_xs[2][MFN_COLS][MF_KC / 32];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+// The tiled form, for many columns per weight row: a block of four waves (2
+// x 2) computes 32 RT weight rows x 32 CT token columns, a wave 16 RT x 16 CT
+// (RT x CT MFMA tiles per group, whose operands are read from LDS RT + CT
+// times).  K goes through LDS in stages of 128 bytes (four groups) in four
+// buffers, loaded by the LDS direct loads (no registers, no store
+// instructions), three stages ahead.  A direct load's wave writes 64
+// consecutive 16-byte pieces, so a stage's rows lie unpadded and their pieces
+// are permuted instead: piece p of row r is at p ^ ((r >> 1) & 7), and the 16
+// rows of an operand read fall on different banks.
+//
+// The fold takes the MFMA's result as a float without a conversion: the
+// accumulator starts from the bits of 1.5 * 2^23, to which the integer sum
+// |acc| <= 32 * 128 * 127 < 2^22 is added in the float's last places, and
+// subtracting 1.5 * 2^23 leaves float(acc) exactly (a conversion takes twice
+// a subtraction's cycles).
+//
+// Same group sums and the same multiply and add per group in order as
+// k_mfma_q8, so the same bits.  K % 128 == 0.
+#define MFT_KC 128
+#define MFT_NB 4
+typedef float v4f_t __attribute__((ext_vector_type(4)));
+typedef const __attribute__((address_space(1))) void *mft_gptr;
+typedef __attribute__((address_space(3))) void *mft_lptr;
+
+// All but the last n of the wave's loads arrived, its LDS reads done, then
+// the block's barrier: the next stage is whole and the buffer before it free.
+template <int N>
+__device__ __forceinline__ void mft_arrive() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
+template <int RT, int CT, int WR, int WC>
+__global__ __launch_bounds__(64 * WR * WC) void k_mfma_q8t(const int8_t *W0, const float *ws0, int N0, int K0,
+                                                           size_t w_group_stride, const int8_t *X0, const float *Xs0,
+                                                           int M, MfCols cols, float *out0, int out_stride0,
+                                                           MfJobs jobs) {
+    constexpr int TR = 16 * RT * WR, TC = 16 * CT * WC;   // the block's tile
+    constexpr int NTHR = 64 * WR * WC, PW = TR * 8 / NTHR, PX = TC * 8 / NTHR, SL = TC / (WR * WC);
+    static_assert(TR * 8 % NTHR == 0 && TC * 8 % NTHR == 0 && SL <= 64, "whole direct loads");
+    constexpr int LPS = PW + PX + 1;                      // direct loads of a wave per stage
+    // a buffer: weight rows, activation columns, column scales.  One array: of
+    // several the compiler would know which a direct load fills, and wait for
+    // all loads in flight before reading any
+    constexpr int XO = TR * MFT_KC, SO = XO + TC * MFT_KC, BUF = SO + TC * 16;
+    __shared__ __align__(16) int8_t s_buf[MFT_NB][BUF];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    int bx = blockIdx.x, cy = blockIdx.y, cys = gridDim.y;
+    if (!cols.list) {
+        // Dense: a 1-D grid over row tiles x column tiles.  Block L runs on XCD
+        // L % 8; XCD x takes the x-th eighth of the tiles, columns innermost, so
+        // the column tiles of a weight tile share an L2.
+        const int nct = (M + TC - 1) / TC;
+        const int nrt = jobs.n ? jobs.j[jobs.n - 1].blk0 + (jobs.j[jobs.n - 1].N + TR - 1) / TR : (N0 + TR - 1) / TR;
+        const int per = gridDim.x >> 3, tile = (bx & 7) * per + (bx >> 3);
+        if (tile >= nrt * nct) return;
+        bx = tile / nct;
+        cy = tile - bx * nct;
+        cys = nct;
+    }
     const int8_t *W = W0;
     const float *ws = ws0;
     float *out = out0;
     const int8_t *X = X0;
     const float *Xs = Xs0;
-    int N = N0, K = K0, out_stride = out_stride0, bx = blockIdx.x;
-    int cy = blockIdx.y, cys = gridDim.y;
-    if (!cols.list) {
-        // Dense: a 1-D grid of (row tiles rounded up to 8) x column tiles.
-        // Blocks go to the 8 XCDs in turn by linear index, so block L runs on
-        // XCD L % 8; give XCD x the row tiles x, x + 8, ... with all their
-        // column tiles one after another, so the column tiles that share a
-        // weight tile share that XCD's L2 (weights read from HBM once).
-        const int ny = (M + MFN_COLS - 1) / MFN_COLS, xcd = bx & 7, sl = bx >> 3, q = sl / ny;
-        bx = q * 8 + xcd;
-        cy = sl - q * ny;
-        cys = ny;
-        const int nrt = jobs.n ? jobs.j[jobs.n - 1].blk0 + (jobs.j[jobs.n - 1].N + MFN_ROWS - 1) / MFN_ROWS
-                               : (N0 + MFN_ROWS - 1) / MFN_ROWS;
-        if (bx >= nrt) return;
-    }
+    int N = N0, K = K0, out_stride = out_stride0;
     if (jobs.n) {
         int ji = 0;
 #pragma unroll
@@ -388,80 +371,140 @@ __global__ __launch_bounds__(MF_THREADS) void k_mfma_q8n(const int8_t *__restric
         Wg = W + (size_t)e * w_group_stride;
         wsg = ws + (size_t)e * N;
     }
-    const int n0 = bx * MFN_ROWS, nb = K >> 5;
-    const int pc = tid & 15, rr = tid >> 4;
-    auto wrow = [&](int j) { const int r = n0 + rr + 16 * j; return Wg + (size_t)(r < N ? r : N - 1) * K; };
-    const int8_t *wl0 = wrow(0), *wl1 = wrow(1), *wl2 = wrow(2), *wl3 = wrow(3);
-    const int kq = 8 * (lane >> 4);
-    const int nst = (K + MF_KC - 1) / MF_KC;
+    const int n0 = bx * TR, nb = K >> 5, nst = K / MFT_KC;
+    // this thread's pieces of a stage: rows i NTHR / 8 + tid / 8, LDS place
+    // tid % 8 (the row's bits 1..3 do not depend on i)
+    const int prow = tid >> 3, gp = 16 * ((tid & 7) ^ ((prow >> 1) & 7));
+    uint32_t wl[PW];
+#pragma unroll
+    for (int i = 0; i < PW; i++) wl[i] = (uint32_t)imin(n0 + NTHR / 8 * i + prow, N - 1) * (uint32_t)K + gp;
+    // operand reads: lane l's 8 bytes 8 (l / 16) of group g of row l % 16
+    const int r16 = lane & 15, q = lane >> 4;
+    const int wr0 = (wave % WR) * 16 * RT, wc0 = (wave / WR) * 16 * CT;
+    int oa[4], ox[4];
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+        const int o = r16 * MFT_KC + 16 * ((2 * g + (q >> 1)) ^ (r16 >> 1)) + 8 * (q & 1);
+        oa[g] = wr0 * MFT_KC + o;
+        ox[g] = XO + wc0 * MFT_KC + o;
+    }
+    const int os = SO + (wc0 + r16) * 16;
 #pragma unroll 1
-    for (int c0 = cy * MFN_COLS; c0 < ncols; c0 += cys * MFN_COLS) {
+    for (int c0 = cy * TC; c0 < ncols; c0 += cys * TC) {
         auto xrow = [&](int c) {
             const int cc = imin(c0 + c, ncols - 1);
             if (!cols.list) return cc;
             const int o = cols.list[cbase + cc];
             return cols.xmap ? cols.xmap[o] : o;
         };
-        const int8_t *xl0 = X + (size_t)xrow(rr) * K;                  // column rr's piece pc
-        const float *xsl = Xs + (size_t)xrow(tid >> 2) * nb;            // threads < 64: column tid / 4
-        const int cl = c0 + (lane & 15);
-        int4 Aw0, Aw1, Aw2, Aw3, Ax0, Bw0, Bw1, Bw2, Bw3, Bx0;
-        float At0 = 0.0f, At1 = 0.0f, Bt0 = 0.0f, Bt1 = 0.0f;
-        float f[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        const bool one = nb == 1;
-        float s0 = 0.0f;
-        auto compute = [&](int buf, int st) {
-            const float *sc = s_xs[buf][lane & 15];
-            const v4i_t zero = {0, 0, 0, 0};
-            const int ng = FULLK ? MF_KC / 32 : nb - st * (MF_KC / 32);
+        // offsets from the uniform bases, so that a load takes no address
+        // arithmetic (a weight matrix and the rows are below 4 GiB each)
+        uint32_t xl[PX];
 #pragma unroll
-            for (int gl = 0; gl < MF_KC / 32; gl++) {
-                if (!FULLK && gl >= ng) break;                     // uniform
-                const long b = *reinterpret_cast<const long *>(&s_x[buf][lane & 15][32 * gl + kq]);
-                const long a = *reinterpret_cast<const long *>(&s_w[buf][16 * wave + (lane & 15)][32 * gl + kq]);
-                const v4i_t dd = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b, zero, 0, 0, 0);
-                mf_fold(f, dd, sc[gl], one);
-            }
-            if (!FULLK && one) s0 = sc[0];
+        for (int i = 0; i < PX; i++) xl[i] = (uint32_t)xrow(NTHR / 8 * i + prow) * (uint32_t)K + gp;
+        // group scales: lanes below SL of each wave, a column's four each
+        const uint32_t xsl = (uint32_t)xrow(wave * SL + imin(lane, SL - 1)) * (uint32_t)nb * 4;
+        auto issue = [&](int st, int b) {
+            const int8_t *wb = Wg + (size_t)st * MFT_KC, *xb = X + (size_t)st * MFT_KC;
+            const int8_t *sb = reinterpret_cast<const int8_t *>(Xs) + (size_t)st * 16;
+#pragma unroll
+            for (int i = 0; i < PW; i++)
+                __builtin_amdgcn_global_load_lds((mft_gptr)(wb + wl[i]),
+                                                 (mft_lptr)(&s_buf[b][(NTHR * i + 64 * wave) * 16]), 16, 0, 0);
+#pragma unroll
+            for (int i = 0; i < PX; i++)
+                __builtin_amdgcn_global_load_lds((mft_gptr)(xb + xl[i]),
+                                                 (mft_lptr)(&s_buf[b][XO + (NTHR * i + 64 * wave) * 16]), 16, 0, 0);
+            if (lane < SL)
+                __builtin_amdgcn_global_load_lds((mft_gptr)(sb + xsl), (mft_lptr)(&s_buf[b][SO + wave * SL * 16]), 16,
+                                                 0, 0);
         };
-        // stage st in buffer st % 2; the loads of stages st + 1 and st + 2
-        // in flight while it runs (stages past the last reload the last)
-        MFN_STAGE_LOAD(A, 0);
-        MFN_STAGE_PUT(A, 0);
-        __syncthreads();
-        MFN_STAGE_LOAD(A, imin(1, nst - 1));
-#pragma unroll 1
-        for (int st = 0; st < nst; st += 2) {
-            MFN_STAGE_LOAD(B, imin(st + 2, nst - 1));
-            __builtin_amdgcn_sched_barrier(0);
-            compute(0, st);
-            MFN_STAGE_PUT(A, 1);
-            __syncthreads();
-            if (st + 1 >= nst) break;                          // uniform
-            MFN_STAGE_LOAD(A, imin(st + 3, nst - 1));
-            __builtin_amdgcn_sched_barrier(0);
-            compute(1, st + 1);
-            MFN_STAGE_PUT(B, 0);
-            __syncthreads();
-        }
-        if (cl < ncols) {
-            float *op = out + (size_t)(cols.list ? cols.list[cbase + cl] : cl) * out_stride;
+        float f[RT][CT][4];
 #pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int n = n0 + 16 * wave + 4 * (lane >> 4) + v;
-                if (n < N) {
-                    float sum = 0.0f;
-                    if (one) sum = epi_one_group((int)f[v], s0, wsg[n]);
-                    else sum += f[v] * wsg[n];
-                    op[n] = sum;
+        for (int i = 0; i < RT; i++)
+#pragma unroll
+            for (int j = 0; j < CT; j++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) f[i][j][v] = 0.0f;
+        v4i_t magic = {0x4B400000, 0x4B400000, 0x4B400000, 0x4B400000};     // 1.5 * 2^23
+        asm volatile("" : "+v"(magic));                   // (kept in registers)
+        auto compute = [&](int b) {
+            const int8_t *p = s_buf[b];
+            long ka[4][RT], kx[4][CT];
+            v4f_t sc[CT];
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+#pragma unroll
+                for (int i = 0; i < RT; i++) ka[g][i] = *reinterpret_cast<const long *>(p + oa[g] + 16 * i * MFT_KC);
+#pragma unroll
+                for (int j = 0; j < CT; j++) kx[g][j] = *reinterpret_cast<const long *>(p + ox[g] + 16 * j * MFT_KC);
+                if (g == 0)
+#pragma unroll
+                    for (int j = 0; j < CT; j++) sc[j] = *reinterpret_cast<const v4f_t *>(p + os + 256 * j);
+            }
+            v4i_t d[2][RT][CT];
+#pragma unroll
+            for (int i = 0; i < RT; i++)
+#pragma unroll
+                for (int j = 0; j < CT; j++)
+                    d[0][i][j] = __builtin_amdgcn_mfma_i32_16x16x32_i8(ka[0][i], kx[0][j], magic, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            // a group's fold runs beside the next group's MFMAs
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+#pragma unroll
+                for (int i = 0; i < RT; i++)
+#pragma unroll
+                    for (int j = 0; j < CT; j++) {
+                        if (g < 3)
+                            d[(g + 1) & 1][i][j] =
+                                __builtin_amdgcn_mfma_i32_16x16x32_i8(ka[g + 1][i], kx[g + 1][j], magic, 0, 0, 0);
+#pragma unroll
+                        for (int v = 0; v < 4; v++)
+                            f[i][j][v] += (__int_as_float(d[g & 1][i][j][v]) - 12582912.0f) * sc[j][g];
+                        if (g < 3) __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);      // one MFMA,
+                        __builtin_amdgcn_sched_group_barrier(0x002, 12, 0);                // a tile's fold
+                    }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        issue(0, 0);
+        if (nst > 1) issue(1, 1);
+        if (nst > 2) issue(2, 2);
+        // (four stages per turn: the buffers are constants, LDS addresses
+        // immediates)
+#pragma unroll 1
+        for (int st0 = 0; st0 < nst; st0 += MFT_NB) {
+#pragma unroll
+            for (int b = 0; b < MFT_NB; b++) {
+                const int st = st0 + b;
+                if (st >= nst) break;
+                if (st + 2 < nst) mft_arrive<2 * LPS>();
+                else if (st + 1 < nst) mft_arrive<LPS>();
+                else mft_arrive<0>();
+                if (st + 3 < nst) issue(st + 3, (b + 3) & (MFT_NB - 1));
+                compute(b);
+            }
+        }
+        // lane l: rows 4 (l / 16) .. + 3 of a tile, column l % 16
+#pragma unroll
+        for (int j = 0; j < CT; j++) {
+            const int cl = c0 + wc0 + 16 * j + r16;
+            if (cl < ncols) {
+                float *op = out + (size_t)(cols.list ? cols.list[cbase + cl] : cl) * out_stride;
+#pragma unroll
+                for (int i = 0; i < RT; i++) {
+                    const int n = n0 + wr0 + 16 * i + 4 * q;
+#pragma unroll
+                    for (int v = 0; v < 4; v++)
+                        if (n + v < N) op[n + v] = 0.0f + f[i][j][v] * wsg[n + v];
                 }
             }
         }
+        // another tile of this block: its loads wait for every wave's reads
+        if (c0 + cys * TC < ncols) mft_arrive<0>();
     }
 }
-#undef MFN_STAGE_LOAD
-#undef MFN_STAGE_PUT
-
 
 // ------------------------------------------------------ wide producers ---
 //
@@ -553,137 +596,131 @@ extern "C" int l98k_upload_exp_table_mfma(const float *tab) {
     return (int)hipMemcpyToSymbol(HIP_SYMBOL(c_exp_tab), tab, 32 * sizeof(float));
 }
 
-// Dense: out[t][n] (row stride out_stride) for t < M over activation rows
-// t.  Returns 0, a HIP error, or -1 for shapes outside the kernel.
-extern "C" int l98k_mfma_gemm(const int8_t *W, const float *ws, int N, int K, const int8_t *X, const float *Xs, int M,
-                              float *out, int out_stride, hipStream_t st) {
-    if (N < 1 || M < 1 || K < 32 || (K & 31) || out_stride < N) return -1;
-    MfCols c{};
-    if (M <= MFN_DENSE_MAX) {
-        const int nrt8 = ((N + MFN_ROWS - 1) / MFN_ROWS + 7) & ~7;
-        const dim3 gridn(nrt8 * ((M + MFN_COLS - 1) / MFN_COLS), 1, 1);
-        if (K % MF_KC == 0)
-            hipLaunchKernelGGL(k_mfma_q8n<true>, gridn, dim3(MF_THREADS), 0, st, W, ws, N, K, (size_t)0, X, Xs, M, c,
-                               out, out_stride, MfJobs{});
-        else
-            hipLaunchKernelGGL(k_mfma_q8n<false>, gridn, dim3(MF_THREADS), 0, st, W, ws, N, K, (size_t)0, X, Xs, M, c,
-                               out, out_stride, MfJobs{});
-        return (int)hipGetLastError();
-    }
-    const dim3 grid((N + MF_ROWS - 1) / MF_ROWS, (M + MF_COLS - 1) / MF_COLS, 1);
-    if (K % MF_KC == 0)
-        hipLaunchKernelGGL(k_mfma_q8<true>, grid, dim3(MF_THREADS), 0, st, W, ws, N, K, (size_t)0, X, Xs, M, c, out,
-                           out_stride, MfJobs{});
+// The tile of k_mfma_q8t's launches: 32 weight rows x 16 token columns for at
+// most 16 columns, 64 x 32 where that still leaves MFT_BIG tiles or more (four
+// rounds of the chip's 512 block places), else 32 x 32.  Measured (us, rows x
+// K at that many columns; 32 x 16 / 32 x 32 / 64 x 32 tiles; before, on tiles
+// of 64 x 16 up to 128 columns and 16 x 64 above):
+//     4176 x 1024 at  12:   5.5 /  5.6 /  7.8 (6.8)
+//     2048 x 2048 at 128:   8.3 /  8.1 / 11.8 (9.8)
+//     8336 x 2048 at 128:  16.9 / 16.8 / 16.5 (22.1)
+//   131072 x 2048 at 128:   233 /  201 /  174 (254)
+//     4176 x 1024 at 512:    -  / 17.3 / 17.7 (26.2)
+//     8336 x 2048 at 512:    -  / 45.0 / 42.7 (74.7)
+//     2048 x 2048 at 512:    -  / 13.9 / 13.7 (24.3)
+// 64 x 64 tiles and blocks of eight waves were slower at every shape: too few
+// blocks for the waits of one to be covered by another's work.
+#define MFT_BIG 2048
+enum { MFT_32x16, MFT_32x32, MFT_64x32 };
+static int mft_tile_rows(int t) { return t == MFT_64x32 ? 64 : 32; }
+static int mft_tile_cols(int t) { return t == MFT_32x16 ? 16 : 32; }
+static void mft_launch(int t, dim3 grid, const int8_t *W, const float *ws, int N, int K, size_t w_group_stride,
+                       const int8_t *X, const float *Xs, int M, const MfCols &c, float *out, int out_stride,
+                       const MfJobs &jobs, hipStream_t st) {
+    if (t == MFT_32x16)
+        hipLaunchKernelGGL((k_mfma_q8t<1, 1, 2, 1>), grid, dim3(128), 0, st, W, ws, N, K, w_group_stride, X, Xs, M, c,
+                           out, out_stride, jobs);
+    else if (t == MFT_32x32)
+        hipLaunchKernelGGL((k_mfma_q8t<1, 1, 2, 2>), grid, dim3(256), 0, st, W, ws, N, K, w_group_stride, X, Xs, M, c,
+                           out, out_stride, jobs);
     else
-        hipLaunchKernelGGL(k_mfma_q8<false>, grid, dim3(MF_THREADS), 0, st, W, ws, N, K, (size_t)0, X, Xs, M, c, out,
-                           out_stride, MfJobs{});
-    return (int)hipGetLastError();
+        hipLaunchKernelGGL((k_mfma_q8t<2, 1, 2, 2>), grid, dim3(256), 0, st, W, ws, N, K, w_group_stride, X, Xs, M, c,
+                           out, out_stride, jobs);
+}
+// k_mfma_q8t takes offsets of 32 bits into a weight matrix and into the rows.
+static bool mft_ok(int N, int K, int rows) {
+    return K % MFT_KC == 0 && (uint64_t)N * K < (1ull << 32) && (uint64_t)rows * K < (1ull << 32);
 }
 
 // Several dense GEMMs over the same M rows in one launch: job j multiplies
 // W[j] (N[j] x K[j], scales ws[j]) over the rows of X[j] / Xs[j] into out[j]
 // (row stride out_stride[j]).  The blocks of job j follow those of job
-// j - 1.  The full-stage instance needs every K a multiple of 256.
+// j - 1.  Returns 0, a HIP error, or -1 for shapes outside the kernels.
 extern "C" int l98k_mfma_gemm_multi(int n_jobs, const int8_t *const *W, const float *const *ws, const int *N,
                                     float *const *out, const int *out_stride, const int *K,
                                     const int8_t *const *X, const float *const *Xs, int M, hipStream_t st) {
     if (n_jobs < 1 || n_jobs > MF_MAX_JOBS || M < 1) return -1;
-    const bool narrow = M <= MFN_DENSE_MAX;
-    const int tile = narrow ? MFN_ROWS : MF_ROWS;
-    MfJobs jobs{};
-    int blocks = 0;
-    bool full = true;
+    bool tiled = true;
+    size_t rows = 0;
     for (int j = 0; j < n_jobs; j++) {
         if (N[j] < 1 || out_stride[j] < N[j] || K[j] < 32 || (K[j] & 31)) return -1;
-        full = full && K[j] % MF_KC == 0;
+        tiled = tiled && mft_ok(N[j], K[j], M);
+        rows += (size_t)N[j];
+    }
+    int t = M <= 16 ? MFT_32x16 : MFT_32x32;
+    if (M > 16 && (rows / 64) * ((M + 31) / 32) >= MFT_BIG) t = MFT_64x32;
+    const int tr = tiled ? mft_tile_rows(t) : MF_ROWS;
+    MfJobs jobs{};
+    int blocks = 0;
+    for (int j = 0; j < n_jobs; j++) {
         jobs.j[j] = MfJob{W[j], ws[j], out[j], X[j], Xs[j], N[j], out_stride[j], blocks, K[j]};
-        blocks += (N[j] + tile - 1) / tile;
+        blocks += (N[j] + tr - 1) / tr;
     }
-    jobs.n = n_jobs;
-    MfCols c{};
-    if (narrow) {
-        const dim3 gridn(((blocks + 7) & ~7) * ((M + MFN_COLS - 1) / MFN_COLS), 1, 1);
-        if (full)
-            hipLaunchKernelGGL(k_mfma_q8n<true>, gridn, dim3(MF_THREADS), 0, st, W[0], ws[0], N[0], K[0], (size_t)0,
-                               X[0], Xs[0], M, c, out[0], out_stride[0], jobs);
-        else
-            hipLaunchKernelGGL(k_mfma_q8n<false>, gridn, dim3(MF_THREADS), 0, st, W[0], ws[0], N[0], K[0], (size_t)0,
-                               X[0], Xs[0], M, c, out[0], out_stride[0], jobs);
-        return (int)hipGetLastError();
+    jobs.n = n_jobs > 1 ? n_jobs : 0;               // one GEMM: the launch's own arguments
+    if (tiled) {
+        const int tiles = blocks * ((M + mft_tile_cols(t) - 1) / mft_tile_cols(t));
+        mft_launch(t, dim3((tiles + 7) & ~7), W[0], ws[0], N[0], K[0], 0, X[0], Xs[0], M, MfCols{}, out[0],
+                   out_stride[0], jobs, st);
+    } else {
+        hipLaunchKernelGGL(k_mfma_q8, dim3(blocks, (M + MF_COLS - 1) / MF_COLS), dim3(MF_THREADS), 0, st, W[0], ws[0],
+                           N[0], K[0], (size_t)0, X[0], Xs[0], M, MfCols{}, out[0], out_stride[0], jobs);
     }
-    const dim3 grid(blocks, (M + MF_COLS - 1) / MF_COLS, 1);
-    if (full)
-        hipLaunchKernelGGL(k_mfma_q8<true>, grid, dim3(MF_THREADS), 0, st, W[0], ws[0], N[0], K[0], (size_t)0, X[0],
-                           Xs[0], M, c, out[0], out_stride[0], jobs);
-    else
-        hipLaunchKernelGGL(k_mfma_q8<false>, grid, dim3(MF_THREADS), 0, st, W[0], ws[0], N[0], K[0], (size_t)0, X[0],
-                           Xs[0], M, c, out[0], out_stride[0], jobs);
     return (int)hipGetLastError();
+}
+
+// Dense: out[t][n] (row stride out_stride) for t < M over activation rows t.
+extern "C" int l98k_mfma_gemm(const int8_t *W, const float *ws, int N, int K, const int8_t *X, const float *Xs, int M,
+                              float *out, int out_stride, hipStream_t st) {
+    return l98k_mfma_gemm_multi(1, &W, &ws, &N, &out, &out_stride, &K, &X, &Xs, M, st);
 }
 
 // Grouped (experts): group g (< *ng <= max_groups) multiplies bank rows of
 // expert gexp[g] with its columns list[goff[g] ..], at most max_cols each.
-// Groups of about 16 columns or fewer (mean_cols, the caller's estimate)
-// take the 64-row x 16-column tiles, larger ones the 16 x 64 tiles.
+// mean_cols, the caller's estimate of a group's columns, picks 16 or 32
+// columns per tile; a group's tiles spread over the grid's y, about twice the
+// mean's (blocks past a group's tiles exit at once, the tiles past the grid
+// are walked).  With bank3, two GEMMs over the same columns and groups (an
+// expert's w1 and w3 banks, both N x K) as jobs of one launch.
+static int mf_grouped(const int8_t *bank, const float *bank_s, float *out, const int8_t *bank3, const float *bank3_s,
+                      float *out3, int N, int K, const int8_t *X, const float *Xs, const int *ng, int max_groups,
+                      const int *gexp, const int *goff, const int *gcnt, const int *list, const int *xmap,
+                      int max_cols, int mean_cols, int out_stride, hipStream_t st) {
+    if (N < 1 || K < 32 || (K & 31) || max_groups < 1 || max_cols < 1 || out_stride < N) return -1;
+    const MfCols c{gexp, goff, gcnt, list, xmap, ng};
+    const bool tiled = mft_ok(N, K, max_cols * MAX_TOPK);
+    const int t = mean_cols <= 16 ? MFT_32x16 : MFT_32x32, tr = tiled ? mft_tile_rows(t) : MF_ROWS;
+    const int nrt = (N + tr - 1) / tr;
+    MfJobs jobs{};
+    if (bank3) {
+        jobs.j[0] = MfJob{bank, bank_s, out, X, Xs, N, out_stride, 0, K};
+        jobs.j[1] = MfJob{bank3, bank3_s, out3, X, Xs, N, out_stride, nrt, K};
+        jobs.n = 2;
+    }
+    if (tiled) {
+        const int tc = mft_tile_cols(t), most = (max_cols + tc - 1) / tc, ys = 2 + 2 * mean_cols / tc;
+        mft_launch(t, dim3(bank3 ? 2 * nrt : nrt, ys < most ? ys : most, max_groups), bank, bank_s, N, K, (size_t)N * K,
+                   X, Xs, 0, c, out, out_stride, jobs, st);
+    } else {
+        hipLaunchKernelGGL(k_mfma_q8, dim3(bank3 ? 2 * nrt : nrt, 1, max_groups), dim3(MF_THREADS), 0, st, bank,
+                           bank_s, N, K, (size_t)N * K, X, Xs, 0, c, out, out_stride, jobs);
+    }
+    return (int)hipGetLastError();
+}
 extern "C" int l98k_mfma_gemm_grouped(const int8_t *bank, const float *bank_s, int N, int K, const int8_t *X,
                                       const float *Xs, const int *ng, int max_groups, const int *gexp,
                                       const int *goff, const int *gcnt, const int *list, const int *xmap,
                                       int max_cols, int mean_cols, float *out, int out_stride, hipStream_t st) {
-    if (N < 1 || K < 32 || (K & 31) || max_groups < 1 || max_cols < 1 || out_stride < N) return -1;
-    MfCols c{gexp, goff, gcnt, list, xmap, ng};
-    if (mean_cols <= MFN_COLS) {
-        const int ys = max_cols > 3 * MFN_COLS ? 4 : (max_cols + MFN_COLS - 1) / MFN_COLS;
-        const dim3 gridn((N + MFN_ROWS - 1) / MFN_ROWS, ys, max_groups);
-        if (K % MF_KC == 0)
-            hipLaunchKernelGGL(k_mfma_q8n<true>, gridn, dim3(MF_THREADS), 0, st, bank, bank_s, N, K, (size_t)N * K, X,
-                               Xs, 0, c, out, out_stride, MfJobs{});
-        else
-            hipLaunchKernelGGL(k_mfma_q8n<false>, gridn, dim3(MF_THREADS), 0, st, bank, bank_s, N, K, (size_t)N * K,
-                               X, Xs, 0, c, out, out_stride, MfJobs{});
-        return (int)hipGetLastError();
-    }
-    const dim3 grid((N + MF_ROWS - 1) / MF_ROWS, 1, max_groups);
-    if (K % MF_KC == 0)
-        hipLaunchKernelGGL(k_mfma_q8<true>, grid, dim3(MF_THREADS), 0, st, bank, bank_s, N, K, (size_t)N * K, X, Xs, 0,
-                           c, out, out_stride, MfJobs{});
-    else
-        hipLaunchKernelGGL(k_mfma_q8<false>, grid, dim3(MF_THREADS), 0, st, bank, bank_s, N, K, (size_t)N * K, X, Xs,
-                           0, c, out, out_stride, MfJobs{});
-    return (int)hipGetLastError();
+    return mf_grouped(bank, bank_s, out, nullptr, nullptr, nullptr, N, K, X, Xs, ng, max_groups, gexp, goff, gcnt,
+                      list, xmap, max_cols, mean_cols, out_stride, st);
 }
-
-// Two grouped GEMMs over the same columns and groups (an expert's w1 and w3
-// banks, both N x K): on the narrow tiles one launch whose first half of
-// block columns runs bank 1 and the second half bank 3 (jobs); otherwise
-// two launches.
 extern "C" int l98k_mfma_gemm_grouped2(const int8_t *bank1, const float *bank1_s, float *out1, const int8_t *bank3,
                                        const float *bank3_s, float *out3, int N, int K, const int8_t *X,
                                        const float *Xs, const int *ng, int max_groups, const int *gexp,
                                        const int *goff, const int *gcnt, const int *list, const int *xmap,
                                        int max_cols, int mean_cols, int out_stride, hipStream_t st) {
-    if (N < 1 || K < 32 || (K & 31) || max_groups < 1 || max_cols < 1 || out_stride < N) return -1;
-    if (mean_cols > MFN_COLS) {
-        const int rc = l98k_mfma_gemm_grouped(bank1, bank1_s, N, K, X, Xs, ng, max_groups, gexp, goff, gcnt, list, xmap,
-                                              max_cols, mean_cols, out1, out_stride, st);
-        if (rc) return rc;
-        return l98k_mfma_gemm_grouped(bank3, bank3_s, N, K, X, Xs, ng, max_groups, gexp, goff, gcnt, list, xmap,
-                                      max_cols, mean_cols, out3, out_stride, st);
-    }
-    MfCols c{gexp, goff, gcnt, list, xmap, ng};
-    const int nrt = (N + MFN_ROWS - 1) / MFN_ROWS;
-    MfJobs jobs{};
-    jobs.j[0] = MfJob{bank1, bank1_s, out1, X, Xs, N, out_stride, 0, K};
-    jobs.j[1] = MfJob{bank3, bank3_s, out3, X, Xs, N, out_stride, nrt, K};
-    jobs.n = 2;
-    const int ys = max_cols > 3 * MFN_COLS ? 4 : (max_cols + MFN_COLS - 1) / MFN_COLS;
-    const dim3 gridn(2 * nrt, ys, max_groups);
-    if (K % MF_KC == 0)
-        hipLaunchKernelGGL(k_mfma_q8n<true>, gridn, dim3(MF_THREADS), 0, st, bank1, bank1_s, N, K, (size_t)N * K, X, Xs,
-                           0, c, out1, out_stride, jobs);
-    else
-        hipLaunchKernelGGL(k_mfma_q8n<false>, gridn, dim3(MF_THREADS), 0, st, bank1, bank1_s, N, K, (size_t)N * K, X, Xs,
-                           0, c, out1, out_stride, jobs);
-    return (int)hipGetLastError();
+    if (!bank3) return -1;
+    return mf_grouped(bank1, bank1_s, out1, bank3, bank3_s, out3, N, K, X, Xs, ng, max_groups, gexp, goff, gcnt, list,
+                      xmap, max_cols, mean_cols, out_stride, st);
 }
 
 static bool wide_pro_ok(int mode, int src_stride, const int *sel_idx, const float *sel_w, int topk, int n, int rows) {
