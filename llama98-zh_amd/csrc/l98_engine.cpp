@@ -810,6 +810,8 @@ struct DState {
     int *amax_tok = nullptr;
     int amax_mode = 0;
     DevCtl *ctl_pinned = nullptr;
+    char *mirrors = nullptr;                // the LZRunState's host mirrors (mirrors_alloc)
+    bool mirrors_pinned = false;
     int cap_rows = 0;                       // rows of hcap / tokbuf
     RoundRec *hist = nullptr;               // device round records
     int hist_cap = 0;
@@ -1017,7 +1019,9 @@ int ctl_put(DState *s, const DevCtl &h) {
     return 0;
 }
 // The host-API entry points that read mtp_chain take the caller's copy:
-// as in the reference, the struct field is the state a caller may set.
+// as in the reference, the struct field is the state a caller may set.  (The
+// field is pinned, so the copy reads it when the stream gets there; every
+// caller waits for the stream before it returns.)
 int chain_put(DState *d, const LZRunState *s) {
     CK(hipMemcpyAsync(d->chain, s->mtp_chain, sizeof(float) * d->m->c.hidden_size, hipMemcpyHostToDevice, d->st));
     return 0;
@@ -1832,6 +1836,51 @@ int mtp_prefill_dev(DState *s, const float *h, const int *toks, int n, const int
 
 }  // namespace
 
+namespace {
+// The run state's host mirrors, zeroed, in one block of pinned memory: a
+// device copy into pageable memory is staged piece by piece on the calling
+// thread (measured: the 67 MB of logits of a 32-session verify of 4 rows at V
+// = 131072 take 4.9 ms, 1.0 MB of a 4-row verify at V = 65536 0.32 ms alone),
+// into pinned memory it runs at the link's rate (1.3 ms and 0.03 ms).
+// Non-coherent (only copies write it, and the stream is waited for before it
+// is read), and cleared by the device: the host's first touch of 2.9 MB takes
+// 1.1 ms of page faults, which it now takes only for the pages it reads.
+// Pageable when the host has no memory to pin.
+bool mirrors_alloc(LZRunState *s, DState *d, const LZModelConfig &c) {
+    const size_t V = (size_t)c.vocab_size, H = (size_t)c.hidden_size, rows = L98_SPEC_K_GPU + 1;
+    size_t off = 0;
+    auto take = [&](size_t floats) { const size_t o = off; off = (off + 4 * floats + 255) & ~(size_t)255; return o; };
+    const size_t ol = take(V), om = take(rows * V), oh = take(rows * H), oc = take(H), od = take(V),
+                 ok = take(c.mtp_n_draft > 1 ? LZ_SPEC_K_MAX * V : 0);
+    d->mirrors_pinned = hipHostMalloc((void **)&d->mirrors, off, hipHostMallocPortable | hipHostMallocNonCoherent) ==
+                        hipSuccess;
+    if (!d->mirrors_pinned) {
+        (void)hipGetLastError();
+        d->mirrors = (char *)malloc(off);
+    }
+    if (!d->mirrors) return false;
+    if (d->mirrors_pinned) {
+        if (hipMemsetAsync(d->mirrors, 0, off, d->st) != hipSuccess || hipStreamSynchronize(d->st) != hipSuccess)
+            return false;
+    } else {
+        memset(d->mirrors, 0, off);
+    }
+    char *b = d->mirrors;
+    s->logits = (float *)(b + ol);
+    s->mtp_logits = (float *)(b + om);
+    s->mtp_verify_hidden = (float *)(b + oh);
+    s->mtp_chain = (float *)(b + oc);
+    s->mtp_draft_logits = (float *)(b + od);
+    s->mtp_kdraft_logits = c.mtp_n_draft > 1 ? (float *)(b + ok) : nullptr;
+    return true;
+}
+void mirrors_free(DState *d) {
+    if (d->mirrors_pinned) (void)hipHostFree(d->mirrors);
+    else free(d->mirrors);
+    d->mirrors = nullptr;
+}
+}  // namespace
+
 extern "C" int lz_state_alloc(LZRunState *s, const LZModel *mm, int seq_len, int spec_k_max,
                               char *errbuf, int errlen) {
     if (!s || !mm || !mm->impl) { set_err(errbuf, errlen, "null argument"); return 1; }
@@ -1872,13 +1921,11 @@ extern "C" int lz_state_alloc(LZRunState *s, const LZModel *mm, int seq_len, int
     s->ssm_ring_depth = d->depth;
     s->nt_cap = 4;
     s->bytes_device = (long long)d->arena_size;
-    s->logits = (float *)calloc((size_t)c.vocab_size, sizeof(float));
-    s->mtp_logits = (float *)calloc((size_t)(L98_SPEC_K_GPU + 1) * c.vocab_size, sizeof(float));
-    s->mtp_verify_hidden = (float *)calloc((size_t)(L98_SPEC_K_GPU + 1) * c.hidden_size, sizeof(float));
-    s->mtp_chain = (float *)calloc((size_t)c.hidden_size, sizeof(float));
-    s->mtp_draft_logits = (float *)calloc((size_t)c.vocab_size, sizeof(float));
-    s->mtp_kdraft_logits = c.mtp_n_draft > 1 ? (float *)calloc((size_t)LZ_SPEC_K_MAX * c.vocab_size, sizeof(float))
-                                             : nullptr;
+    if (!mirrors_alloc(s, d, c)) {
+        set_err(errbuf, errlen, "no host memory for the logits mirrors");
+        lz_state_free(s);
+        return 1;
+    }
     lz_state_reset(s, mm);
     return 0;
 }
@@ -1900,10 +1947,9 @@ extern "C" void lz_state_free(LZRunState *s) {
         for (auto &g : d->temp_graph)
             if (g) (void)hipGraphExecDestroy(g);
         if (d->st) (void)hipStreamDestroy(d->st);
+        mirrors_free(d);
         delete d;
     }
-    free(s->logits); free(s->mtp_logits); free(s->mtp_verify_hidden);
-    free(s->mtp_chain); free(s->mtp_draft_logits); free(s->mtp_kdraft_logits);
     memset(s, 0, sizeof(*s));
 }
 
