@@ -825,11 +825,10 @@ struct DState {
     // temperature sampling scratch (allocated on first use)
     char *smp_arena = nullptr;
     float *smp_q = nullptr;                 // [L98_SPEC_K_GPU][V] draft distributions of a round
-    float *smp_p = nullptr, *smp_probs = nullptr;
+    float *smp_p = nullptr, *smp_probs = nullptr;         // [L98_SPEC_K_GPU + 1][V], as the keys and indices
     uint32_t *smp_keys = nullptr, *smp_skeys = nullptr;
     int *smp_svals = nullptr;
-    void *smp_tmp = nullptr;
-    size_t smp_tmp_bytes = 0;
+    void *smp_tmp = nullptr, *smp_top = nullptr;
     unsigned long long *smp_rng = nullptr;
     int *smp_out = nullptr;                 // [16] small results
     float *smp_outf = nullptr;              // [16]
@@ -2592,18 +2591,19 @@ extern "C" int lz_spec_round(const LZModel *mm, LZRunState *s, int anchor, int a
 namespace {
 
 // The temperature sampling scratch of a state, carved from one allocation
-// on first use: the round's draft distributions, a target distribution, the
-// softmax and the top-p candidate keys/indices (sorted copies too), the
-// sort's scratch, the generator state and small results.
+// on first use: the round's draft distributions, the verify rows' target
+// distributions, softmax and top-p candidate keys/indices (sorted copies
+// too), the sort's scratch, the generator state and small results.
 bool smp_ensure(DState *d) {
     if (d->smp_arena) return true;
     const size_t V = (size_t)d->m->c.vocab_size;
-    const size_t tmp = l98k_smp_sort_tmp_bytes((int)V);
+    const int rows = L98_SPEC_K_GPU + 1;
+    const size_t tmp = l98k_smp_sort_tmp_bytes((int)V, rows), W = 4 * V * (size_t)rows;
     size_t off = 0;
     auto take = [&](size_t bytes) { size_t a = off; off = (off + bytes + 255) & ~(size_t)255; return a; };
-    const size_t oq = take(sizeof(float) * V * L98_SPEC_K_GPU), op = take(sizeof(float) * V),
-                 opr = take(sizeof(float) * V), ok = take(4 * V), osk = take(4 * V),
-                 osv = take(4 * V), ot = take(tmp), orng = take(8), oo = take(64), oof = take(64);
+    const size_t oq = take(sizeof(float) * V * L98_SPEC_K_GPU), op = take(W), opr = take(W), ok = take(W),
+                 osk = take(W), osv = take(W), ot = take(tmp), otp = take(l98k_smp_topp_tmp_bytes(rows)),
+                 orng = take(8), oo = take(64), oof = take(64);
     char *a = nullptr;
     if (hipMalloc(&a, off) != hipSuccess) return false;
     d->smp_arena = a;
@@ -2614,27 +2614,30 @@ bool smp_ensure(DState *d) {
     d->smp_skeys = (uint32_t *)(a + osk);
     d->smp_svals = (int *)(a + osv);
     d->smp_tmp = a + ot;
-    d->smp_tmp_bytes = tmp;
+    d->smp_top = a + otp;
     d->smp_rng = (unsigned long long *)(a + orng);
     d->smp_out = (int *)(a + oo);
     d->smp_outf = (float *)(a + oof);
     return true;
 }
 
-// lz_target_dist (top-k and min-p off, src/sampler.c:682-730) of a device
-// logits row into d->smp_p: softmax(row / T), then with top-p the
+// lz_target_dist (top-k and min-p off, src/sampler.c:682-730) of `rows`
+// device logits rows into d->smp_p (a verify's rows together: none depends on
+// another's acceptance, and each launch's one block per row leaves the chip
+// to the others): softmax(row / T), then with top-p the
 // candidates >= (1 - top_p) / (V - 1) sorted by probability (stable), the
 // prefix up to the first cumulative mass >= top_p renormalized.
 // skip: a device flag (null: never) that turns every launch into a no-op.
-int dev_target_dist(DState *d, const float *row, int V, float temp, float topp, const int *skip = nullptr) {
+int dev_target_dist(DState *d, const float *logits, int rows, int V, float temp, float topp,
+                    const int *skip = nullptr) {
     const float inv = 1.0f / temp;
-    if (!topp_active(topp)) return l98k_smp_softmax(row, V, inv, d->smp_p, 0.0f, nullptr, nullptr, skip, d->st);
+    if (!topp_active(topp)) return l98k_smp_softmax(logits, V, rows, inv, d->smp_p, 0.0f, nullptr, nullptr, skip, d->st);
     const float cutoff = (V > 1) ? (1.0f - topp) / (float)(V - 1) : 0.0f;
-    if (l98k_smp_softmax(row, V, inv, d->smp_probs, cutoff, d->smp_keys, d->smp_out + 8, skip, d->st) ||
-        l98k_smp_sort_desc(d->smp_keys, d->smp_skeys, d->smp_svals, V, d->smp_tmp, skip, d->st))
+    if (l98k_smp_softmax(logits, V, rows, inv, d->smp_probs, cutoff, d->smp_keys, d->smp_out + 8, skip, d->st) ||
+        l98k_smp_sort_desc(d->smp_keys, d->smp_skeys, d->smp_svals, V, rows, d->smp_tmp, skip, d->st))
         return 1;
-    return l98k_smp_topp_dist(d->smp_probs, V, d->smp_skeys, d->smp_svals, d->smp_out + 8, topp, d->smp_p, skip,
-                              d->st);
+    return l98k_smp_topp_dist(d->smp_probs, V, rows, d->smp_skeys, d->smp_svals, d->smp_out + 8, topp, d->smp_top,
+                              d->smp_p, skip, d->st);
 }
 
 // lz_sample_ex for temperature > 0 (src/sampler.c:794-840) on a device
@@ -2644,13 +2647,13 @@ int dev_sample_ex(DState *d, const float *row, int V, float temp, float topp, lz
     const float inv = 1.0f / temp;
     if (hipMemcpyAsync(d->smp_rng, rng, sizeof(lz_u64), hipMemcpyHostToDevice, d->st)) return 1;
     if (!topp_active(topp)) {
-        if (l98k_smp_softmax(row, V, inv, d->smp_probs, 0.0f, nullptr, nullptr, nullptr, d->st) ||
+        if (l98k_smp_softmax(row, V, 1, inv, d->smp_probs, 0.0f, nullptr, nullptr, nullptr, d->st) ||
             l98k_smp_draw(d->smp_probs, V, d->smp_rng, d->smp_out, nullptr, nullptr, nullptr, d->st))
             return 1;
     } else {
         const float cutoff = (V > 1) ? (1.0f - topp) / (float)(V - 1) : 0.0f;
-        if (l98k_smp_softmax(row, V, inv, d->smp_probs, cutoff, d->smp_keys, d->smp_out + 8, nullptr, d->st) ||
-            l98k_smp_sort_desc(d->smp_keys, d->smp_skeys, d->smp_svals, V, d->smp_tmp, nullptr, d->st) ||
+        if (l98k_smp_softmax(row, V, 1, inv, d->smp_probs, cutoff, d->smp_keys, d->smp_out + 8, nullptr, d->st) ||
+            l98k_smp_sort_desc(d->smp_keys, d->smp_skeys, d->smp_svals, V, 1, d->smp_tmp, nullptr, d->st) ||
             l98k_smp_sample_topp(d->smp_probs, V, d->smp_skeys, d->smp_svals, d->smp_out + 8, topp, d->smp_rng,
                                  d->smp_out, d->st))
             return 1;
@@ -2664,8 +2667,8 @@ int dev_sample_ex(DState *d, const float *row, int V, float temp, float topp, lz
 // One temperature round on the device: lz_spec_round_temp with p_min = 0,
 // n_min = 0 and the one-slot head (src/generate.c:1234-1377).  k chained
 // draft steps, each q_i = softmax(logits/T) and a draw into ctl->tok[1+i]
-// (lz_sample_temp_q, src/sampler.c:736-747); the (k+1)-row verify; per
-// row i the target distribution (lz_target_dist) and the acceptance test
+// (lz_sample_temp_q, src/sampler.c:736-747); the (k+1)-row verify; every
+// row's target distribution (lz_target_dist); per row i the acceptance test
 // with residual resampling, which on a rejection records n_accept = i and
 // sets ctl->smp_done, after which every sampling launch of the round does
 // nothing (the reference's loop stops there, drawing nothing more); the
@@ -2680,20 +2683,18 @@ int enqueue_temp_round(DState *d, int k, int max_pos, float temp, float topp) {
     for (int i = 0; i < k; i++) {
         float *qi = d->smp_q + (size_t)i * V;
         CK(draft_step(d, d->ctl->tok + i, &d->ctl->mtp_pos, i, max_pos, d->draft_logits, nullptr));
-        CK(l98k_smp_softmax(d->draft_logits, V, inv, qi, 0.0f, nullptr, nullptr, nullptr, d->st));
+        CK(l98k_smp_softmax(d->draft_logits, V, 1, inv, qi, 0.0f, nullptr, nullptr, nullptr, d->st));
         CK(l98k_smp_draw(qi, V, d->smp_rng, d->smp_out, d->smp_outf, d->ctl->tok + 1 + i, nullptr, d->st));
     }
     CK(forward_chunk(d, d->ctl->tok, k + 1, &d->ctl->anchor_pos, 1, max_pos, d->vhidden, true, d->mtp_logits,
                      false));
     CK(l98k_set_tokens(d->ctl, 2, nullptr, 0, d->st));
     const int *done = &d->ctl->smp_done;
-    for (int i = 0; i < k; i++) {
-        CK(dev_target_dist(d, d->mtp_logits + (size_t)i * V, V, temp, topp, done));
-        CK(l98k_smp_accept_row(d->smp_p, d->smp_q + (size_t)i * V, V, d->ctl->tok + 1 + i, d->smp_rng,
+    CK(dev_target_dist(d, d->mtp_logits, k + 1, V, temp, topp));
+    for (int i = 0; i < k; i++)
+        CK(l98k_smp_accept_row(d->smp_p + (size_t)i * V, d->smp_q + (size_t)i * V, V, d->ctl->tok + 1 + i, d->smp_rng,
                                d->ctl->out + i, &d->ctl->n_accept, &d->ctl->smp_done, i, d->st));
-    }
-    CK(dev_target_dist(d, d->mtp_logits + (size_t)k * V, V, temp, topp, done));
-    CK(l98k_smp_draw(d->smp_p, V, d->smp_rng, d->smp_out, nullptr, d->ctl->out + k, done, d->st));
+    CK(l98k_smp_draw(d->smp_p + (size_t)k * V, V, d->smp_rng, d->smp_out, nullptr, d->ctl->out + k, done, d->st));
     CK(l98k_accept(d->ctl, d->vhidden, c.hidden_size, d->chain, d->depth, 4, d->st));
     if (k > 1) CK(mtp_prefill_dev(d, d->vhidden, d->ctl->catch_tok, k - 1, &d->ctl->catch_pos, 0));
     CK(l98k_set_tokens(d->ctl, 1, d->hist, d->hist_cap, d->st));
@@ -2839,7 +2840,7 @@ int spec_round_temp(const LZModel *mm, LZRunState *s, int anchor, int anchor_pos
         float *qi = d->smp_q + (size_t)i * V;
         int idx = 0;
         float qidx = 0.0f;
-        if (l98k_smp_softmax(row, V, inv, qi, 0.0f, nullptr, nullptr, nullptr, d->st) ||
+        if (l98k_smp_softmax(row, V, 1, inv, qi, 0.0f, nullptr, nullptr, nullptr, d->st) ||
             l98k_smp_draw(qi, V, d->smp_rng, d->smp_out, d->smp_outf, d->ctl->tok + 1 + i, nullptr, d->st) ||
             hipMemcpyAsync(&idx, d->smp_out, sizeof(int), hipMemcpyDeviceToHost, d->st) ||
             hipMemcpyAsync(&qidx, d->smp_outf, sizeof(float), hipMemcpyDeviceToHost, d->st) ||
@@ -2869,18 +2870,17 @@ int spec_round_temp(const LZModel *mm, LZRunState *s, int anchor, int anchor_pos
     // the target distribution of each verify row, then u, then the residual
     // draw on a rejection; the bonus draw when every draft is accepted
     int n_accept = k_eff;
+    if (dev_target_dist(d, d->mtp_logits, k_eff + 1, V, temp, topp)) return -LZ_ERR_FORWARD;
     for (int i = 0; i < k_eff; i++) {
         int res[2] = {0, 0};
-        if (dev_target_dist(d, d->mtp_logits + (size_t)i * V, V, temp, topp) ||
-            l98k_smp_accept(d->smp_p, d->smp_q + (size_t)i * V, V, draft[i], nullptr, d->smp_rng, d->smp_out, d->st) ||
+        if (l98k_smp_accept(d->smp_p + (size_t)i * V, d->smp_q + (size_t)i * V, V, draft[i], nullptr, d->smp_rng, d->smp_out, d->st) ||
             hipMemcpyAsync(res, d->smp_out, sizeof(res), hipMemcpyDeviceToHost, d->st) || hipStreamSynchronize(d->st))
             return -LZ_ERR_FORWARD;
         out[i] = res[0];
         if (!res[1]) { n_accept = i; break; }
     }
     if (n_accept == k_eff) {
-        if (dev_target_dist(d, d->mtp_logits + (size_t)k_eff * V, V, temp, topp) ||
-            l98k_smp_draw(d->smp_p, V, d->smp_rng, d->smp_out, nullptr, nullptr, nullptr, d->st) ||
+        if (l98k_smp_draw(d->smp_p + (size_t)k_eff * V, V, d->smp_rng, d->smp_out, nullptr, nullptr, nullptr, d->st) ||
             hipMemcpyAsync(out + k_eff, d->smp_out, sizeof(int), hipMemcpyDeviceToHost, d->st))
             return -LZ_ERR_FORWARD;
     }
@@ -3056,9 +3056,9 @@ extern "C" int l98_sort_desc(const uint32_t *keys, int n, uint32_t *keys_out, in
         if (keys[i] >= (1u << 30)) return 1;
     DevBuf dk, dko, dio, dt;
     if (!dk.get(keys, sizeof(uint32_t) * (size_t)n) || !dko.get(nullptr, sizeof(uint32_t) * (size_t)n) ||
-        !dio.get(nullptr, sizeof(int) * (size_t)n) || !dt.get(nullptr, l98k_smp_sort_tmp_bytes(n)))
+        !dio.get(nullptr, sizeof(int) * (size_t)n) || !dt.get(nullptr, l98k_smp_sort_tmp_bytes(n, 1)))
         return 1;
-    if (l98k_smp_sort_desc((uint32_t *)dk.p, (uint32_t *)dko.p, (int *)dio.p, n, dt.p, nullptr, nullptr)) return 1;
+    if (l98k_smp_sort_desc((uint32_t *)dk.p, (uint32_t *)dko.p, (int *)dio.p, n, 1, dt.p, nullptr, nullptr)) return 1;
     return dko.put(keys_out, sizeof(uint32_t) * (size_t)n) && dio.put(idx_out, sizeof(int) * (size_t)n) ? 0 : 1;
 }
 

@@ -461,7 +461,9 @@ __device__ __forceinline__ int blk_argmax(const float *x, int n, SmpLds &L) {
 // probs = softmax(logits * inv_t) (the logits scaled in place first, as
 // the reference does); with cutoff > 0 also the top-p candidate keys
 // (order-preserving bits for probs >= cutoff, 0 otherwise) and indices for
-// the descending sort, and their count.
+// the descending sort, and their count.  One block per row of n: a row's
+// passes run at the rate of one CU (68 us at n = 65536), so the rows that a
+// round can know together share a launch.
 __global__ __launch_bounds__(SMP_THREADS) void k_smp_softmax(const float *__restrict__ logits, int n, float inv_t,
                                                              float *__restrict__ probs, float cutoff,
                                                              uint32_t *__restrict__ keys,
@@ -469,6 +471,9 @@ __global__ __launch_bounds__(SMP_THREADS) void k_smp_softmax(const float *__rest
     __shared__ SmpLds L;
     __shared__ float tab[32];
     if (skip && *skip) return;
+    logits += (size_t)blockIdx.x * n;
+    probs += (size_t)blockIdx.x * n;
+    if (keys) keys += (size_t)blockIdx.x * n;
     const int tid = threadIdx.x;
     if (tid < 32) tab[tid] = c_exp_tab[tid];
     uint32_t mk = 0u;
@@ -501,7 +506,7 @@ __global__ __launch_bounds__(SMP_THREADS) void k_smp_softmax(const float *__rest
     if (keys) {
         uint32_t tot = blk_excl_u32(cnt, L) + cnt;
         tot = blk_max_u32(tot, L);
-        if (tid == 0) *n_cand = (int)tot;
+        if (tid == 0) n_cand[blockIdx.x] = (int)tot;
     }
 }
 
@@ -529,27 +534,45 @@ __global__ __launch_bounds__(SMP_THREADS) void k_smp_draw(const float *__restric
 // by probability, descending (stable: ties keep index order): the kept
 // prefix ends at the first cumulative mass >= top_p (or takes every
 // candidate), each kept probability is divided by the kept mass, the rest
-// are 0; no candidate: one-hot at the argmax.
-__global__ __launch_bounds__(SMP_THREADS) void k_smp_topp_dist(const float *__restrict__ probs, int n,
+// are 0; no candidate: one-hot at the argmax.  In two launches: the prefix's
+// end and mass by one block per row, then every element by its sorted place
+// (the sort's indices are a permutation of the row, so the places past the
+// prefix are the zeros).  One block per row writing the row too took 152 us
+// at n = 65536, 90 of them in its scattered stores.
+struct TopP {
+    int last, hot;                       // the prefix's last place (-1: none), the one-hot index (-1: none)
+    float mass;
+    int pad;
+};
+__global__ __launch_bounds__(SMP_THREADS) void k_smp_topp_find(const float *__restrict__ probs, int n,
                                                                const uint32_t *__restrict__ skeys,
-                                                               const int *__restrict__ svals,
                                                                const int *__restrict__ n_cand, float topp,
-                                                               float *__restrict__ p_out, const int *__restrict__ skip) {
+                                                               TopP *__restrict__ out, const int *__restrict__ skip) {
     __shared__ SmpLds L;
     if (skip && *skip) return;
-    const int tid = threadIdx.x, nc = *n_cand;
-    for (int i = tid; i < n; i += SMP_THREADS) p_out[i] = 0.0f;
+    const int tid = threadIdx.x, row = blockIdx.x, nc = n_cand[row];
     if (nc <= 0) {
-        const int a = blk_argmax(probs, n, L);
-        __syncthreads();
-        if (tid == 0) p_out[a] = 1.0f;
+        const int a = blk_argmax(probs + (size_t)row * n, n, L);
+        if (tid == 0) out[row] = TopP{-1, a, 1.0f, 0};
         return;
     }
-    xprefix(GetKeys{skeys, nc}, nc, XP_FIRST_GE, topp * 1.0f, L);
-    const int last = L.result >= 0 ? L.result : nc - 1;
-    const float mass = L.fres;
-    __syncthreads();
-    for (int j = tid; j <= last; j += SMP_THREADS) p_out[svals[j]] = __uint_as_float(skeys[j]) / mass;
+    xprefix(GetKeys{skeys + (size_t)row * n, nc}, nc, XP_FIRST_GE, topp * 1.0f, L);
+    if (tid == 0) out[row] = TopP{L.result >= 0 ? L.result : nc - 1, -1, L.fres, 0};
+}
+#define TOPP_TILE 1024
+__global__ __launch_bounds__(TOPP_TILE) void k_smp_topp_fill(int n, const uint32_t *__restrict__ skeys,
+                                                             const int *__restrict__ svals,
+                                                             const TopP *__restrict__ top, float *__restrict__ p_out,
+                                                             const int *__restrict__ skip) {
+    if (skip && *skip) return;
+    const int j = blockIdx.x * TOPP_TILE + threadIdx.x;
+    if (j >= n) return;
+    const TopP t = top[blockIdx.y];
+    const size_t r = (size_t)blockIdx.y * n;
+    const int i = svals[r + j];
+    float v = j <= t.last ? __uint_as_float(skeys[r + j]) / t.mass : 0.0f;
+    if (i == t.hot) v = 1.0f;
+    p_out[r + i] = v;
 }
 
 // lz_spec_accept_temp on device rows: u (given, or drawn); accept x iff u < min(1,
@@ -646,14 +669,17 @@ __global__ __launch_bounds__(SMP_THREADS) void k_smp_xprefix(const float *__rest
 //
 // Stable descending sort of (key, index) pairs, keys below 2^30: three LSD
 // passes of 10-bit digits over tiles of RS_TILE elements (one per thread,
-// so a tile's elements are in index order across waves and lanes).  A pass
-// is (1) k_rs_count: each tile's digit counts -> hist[digit][tile]; (2)
-// k_rs_scan: the exclusive prefix of hist in (digit, tile) order, by one
-// block; (3) k_rs_scatter: each element to hist[digit][tile] + the count of
-// equal digits before it in its tile (lanes of the same digit found with 10
-// ballots, then the waves before it).  Digits are taken as 1023 - digit, so
-// the order is descending; every pass keeps the order of equal digits, so
-// equal keys keep index order.
+// so a tile's elements are in index order across waves and lanes), over every
+// row at once (the grid's y).  A pass is (1) k_rs_count: each tile's digit
+// counts -> hist[tile][digit]; (2) k_rs_scatter: each block sums the digits'
+// totals and the tiles before its own (coalesced reads of the whole table,
+// 256 KB at n = 65536), scans the totals over the digits, and puts each
+// element at its digit's start + the tiles before + the count of equal digits
+// before it in its tile (lanes of the same digit found with 10 ballots, then
+// the waves before it).  A launch of one block scanning the table between the
+// two took 25 us per pass.  Digits are taken as 1023 - digit, so the order is
+// descending; every pass keeps the order of equal digits, so equal keys keep
+// index order.
 #define RS_TILE 1024
 #define RS_BITS 10
 #define RS_DIG (1 << RS_BITS)
@@ -671,70 +697,9 @@ __global__ __launch_bounds__(RS_TILE) void k_rs_count(const uint32_t *__restrict
     const int tid = threadIdx.x, i = blockIdx.x * RS_TILE + tid;
     cnt[tid] = 0;
     __syncthreads();
-    if (i < n) atomicAdd(&cnt[rs_digit(keys[i], shift)], 1);
+    if (i < n) atomicAdd(&cnt[rs_digit(keys[(size_t)blockIdx.y * n + i], shift)], 1);
     __syncthreads();
-    hist[(size_t)tid * ntiles + blockIdx.x] = cnt[tid];
-}
-
-// Exclusive prefix, in place, of the RS_DIG x ntiles counts in (digit,
-// tile) order: thread t takes digit t's row of ntiles counts (its loads
-// eight 16-byte vectors at a time when ntiles % 4 == 0).
-__global__ __launch_bounds__(RS_TILE) void k_rs_scan(int *__restrict__ hist, int ntiles, const int *__restrict__ skip) {
-    __shared__ int wsum[RS_TILE / 64];
-    if (skip && *skip) return;
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    int *row = hist + (size_t)tid * ntiles;
-    int sum = 0;
-    if ((ntiles & 3) == 0) {
-        const int4 *r4 = reinterpret_cast<const int4 *>(row);
-        const int n4 = ntiles >> 2;
-        for (int i0 = 0; i0 < n4; i0 += 8) {
-            int4 v[8];
-#pragma unroll
-            for (int u = 0; u < 8; u++) v[u] = r4[imin(i0 + u, n4 - 1)];
-#pragma unroll
-            for (int u = 0; u < 8; u++)
-                if (i0 + u < n4) sum += v[u].x + v[u].y + v[u].z + v[u].w;
-        }
-    } else {
-        for (int i = 0; i < ntiles; i++) sum += row[i];
-    }
-    const int incl = (int)wave_scan_u32((uint32_t)sum);
-    if (lane == 63) wsum[w] = incl;
-    __syncthreads();
-    if (w == 0) {
-        int v = lane < RS_TILE / 64 ? wsum[lane] : 0;
-        v = (int)wave_scan_u32((uint32_t)v);
-        if (lane < RS_TILE / 64) wsum[lane] = v;
-    }
-    __syncthreads();
-    int run = (w ? wsum[w - 1] : 0) + incl - sum;
-    if ((ntiles & 3) == 0) {
-        int4 *r4 = reinterpret_cast<int4 *>(row);
-        const int n4 = ntiles >> 2;
-        for (int i0 = 0; i0 < n4; i0 += 8) {
-            int4 v[8];
-#pragma unroll
-            for (int u = 0; u < 8; u++) v[u] = r4[imin(i0 + u, n4 - 1)];
-#pragma unroll
-            for (int u = 0; u < 8; u++) {
-                if (i0 + u < n4) {
-                    int4 o;
-                    o.x = run; run += v[u].x;
-                    o.y = run; run += v[u].y;
-                    o.z = run; run += v[u].z;
-                    o.w = run; run += v[u].w;
-                    r4[i0 + u] = o;
-                }
-            }
-        }
-    } else {
-        for (int i = 0; i < ntiles; i++) {
-            const int c = row[i];
-            row[i] = run;
-            run += c;
-        }
-    }
+    hist[((size_t)blockIdx.y * ntiles + blockIdx.x) * RS_DIG + tid] = cnt[tid];
 }
 
 __global__ __launch_bounds__(RS_TILE) void k_rs_scatter(const uint32_t *__restrict__ keys, const int *__restrict__ vals,
@@ -742,13 +707,35 @@ __global__ __launch_bounds__(RS_TILE) void k_rs_scatter(const uint32_t *__restri
                                                         int n, int shift, const int *__restrict__ hist, int ntiles,
                                                         const int *__restrict__ skip) {
     __shared__ unsigned short wcnt[RS_TILE / 64][RS_DIG];   // per wave: elements of each digit
+    __shared__ int base[RS_DIG], wsum[RS_TILE / 64];
     if (skip && *skip) return;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, i = blockIdx.x * RS_TILE + tid;
     const bool valid = i < n;
+    const size_t row = (size_t)blockIdx.y * n;
+    keys += row;
+    keys_out += row;
+    vals_out += row;
+    if (vals) vals += row;
+    hist += (size_t)blockIdx.y * ntiles * RS_DIG;
     const uint32_t key = valid ? keys[i] : 0u;
     const int val = valid ? (vals ? vals[i] : i) : 0;
     const int dg = rs_digit(key, shift);
     for (int j = tid; j < (RS_TILE / 64) * RS_DIG; j += RS_TILE) (&wcnt[0][0])[j] = 0;
+    // thread t: digit t's total and its count in the tiles before this one
+    int total = 0, before = 0;
+#pragma unroll 1
+    for (int t0 = 0; t0 < ntiles; t0 += 16) {
+        int c[16];
+#pragma unroll
+        for (int u = 0; u < 16; u++) c[u] = hist[(size_t)imin(t0 + u, ntiles - 1) * RS_DIG + tid];
+#pragma unroll
+        for (int u = 0; u < 16; u++) {
+            if (t0 + u < ntiles) total += c[u];
+            if (t0 + u < (int)blockIdx.x) before += c[u];
+        }
+    }
+    const int incl = (int)wave_scan_u32((uint32_t)total);
+    if (lane == 63) wsum[w] = incl;
     // the lanes of this wave holding the same digit
     unsigned long long peers = __ballot(valid);
 #pragma unroll
@@ -759,7 +746,13 @@ __global__ __launch_bounds__(RS_TILE) void k_rs_scatter(const uint32_t *__restri
     const int rank = __popcll(peers & ((1ull << lane) - 1ull));
     __syncthreads();
     if (valid && rank == 0) wcnt[w][dg] = (unsigned short)__popcll(peers);
+    if (w == 0) {
+        int v = lane < RS_TILE / 64 ? wsum[lane] : 0;
+        v = (int)wave_scan_u32((uint32_t)v);
+        if (lane < RS_TILE / 64) wsum[lane] = v;
+    }
     __syncthreads();
+    base[tid] = (w ? wsum[w - 1] : 0) + incl - total + before;
     // thread t: digit t's running count over the waves, exclusive
     {
         int run = 0;
@@ -772,7 +765,7 @@ __global__ __launch_bounds__(RS_TILE) void k_rs_scatter(const uint32_t *__restri
     }
     __syncthreads();
     if (valid) {
-        const int pos = hist[(size_t)dg * ntiles + blockIdx.x] + wcnt[w][dg] + rank;
+        const int pos = base[dg] + wcnt[w][dg] + rank;
         keys_out[pos] = key;
         vals_out[pos] = val;
     }
@@ -784,10 +777,10 @@ extern "C" int l98k_upload_exp_table_smp(const float *tab) {
     return (int)hipMemcpyToSymbol(HIP_SYMBOL(c_exp_tab), tab, 32 * sizeof(float));
 }
 
-extern "C" int l98k_smp_softmax(const float *logits, int n, float inv_t, float *probs, float cutoff, uint32_t *keys,
-                                int *n_cand, const int *skip, hipStream_t st) {
-    if (n < 1) return -1;
-    hipLaunchKernelGGL(k_smp_softmax, dim3(1), dim3(SMP_THREADS), 0, st, logits, n, inv_t, probs, cutoff, keys, n_cand,
+extern "C" int l98k_smp_softmax(const float *logits, int n, int rows, float inv_t, float *probs, float cutoff,
+                                uint32_t *keys, int *n_cand, const int *skip, hipStream_t st) {
+    if (n < 1 || rows < 1) return -1;
+    hipLaunchKernelGGL(k_smp_softmax, dim3(rows), dim3(SMP_THREADS), 0, st, logits, n, inv_t, probs, cutoff, keys, n_cand,
                        skip);
     return (int)hipGetLastError();
 }
@@ -799,20 +792,20 @@ extern "C" int l98k_smp_draw(const float *p, int n, unsigned long long *rng, int
     return (int)hipGetLastError();
 }
 
-extern "C" size_t l98k_smp_sort_tmp_bytes(int n) {
+extern "C" size_t l98k_smp_sort_tmp_bytes(int n, int rows) {
     const size_t ntiles = ((size_t)n + RS_TILE - 1) / RS_TILE;
-    return sizeof(int) * RS_DIG * ntiles + 2 * sizeof(int) * (size_t)n;
+    return sizeof(int) * (RS_DIG * ntiles + (size_t)n) * (size_t)rows;
 }
 
-// Stable descending sort of n keys (below 2^30) with their indices 0..n-1:
-// keys_out, vals_out.  keys is overwritten (a pass's buffer); tmp holds
-// l98k_smp_sort_tmp_bytes(n) bytes.
-extern "C" int l98k_smp_sort_desc(uint32_t *keys, uint32_t *keys_out, int *vals_out, int n, void *tmp,
+// Stable descending sort of each of `rows` rows of n keys (below 2^30) with
+// their indices 0..n-1: keys_out, vals_out.  keys is overwritten (a pass's
+// buffer); tmp holds l98k_smp_sort_tmp_bytes(n, rows) bytes.
+extern "C" int l98k_smp_sort_desc(uint32_t *keys, uint32_t *keys_out, int *vals_out, int n, int rows, void *tmp,
                                   const int *skip, hipStream_t st) {
-    if (n < 1 || n > RS_DIG * RS_TILE || !tmp) return -1;
+    if (n < 1 || n > RS_DIG * RS_TILE || rows < 1 || !tmp) return -1;
     const int ntiles = (n + RS_TILE - 1) / RS_TILE;
     int *hist = reinterpret_cast<int *>(tmp);
-    int *vtmp = hist + (size_t)RS_DIG * ntiles;
+    int *vtmp = hist + (size_t)RS_DIG * ntiles * rows;
     // pass 0: keys -> keys_out (indices implicit) -> vals_out; pass 1:
     // keys_out -> keys, vals_out -> vtmp; pass 2: keys -> keys_out, vtmp ->
     // vals_out
@@ -822,18 +815,24 @@ extern "C" int l98k_smp_sort_desc(uint32_t *keys, uint32_t *keys_out, int *vals_
     int *vout[RS_PASSES] = {vals_out, vtmp, vals_out};
     for (int pass = 0; pass < RS_PASSES; pass++) {
         const int shift = pass * RS_BITS;
-        hipLaunchKernelGGL(k_rs_count, dim3(ntiles), dim3(RS_TILE), 0, st, kin[pass], n, shift, hist, ntiles, skip);
-        hipLaunchKernelGGL(k_rs_scan, dim3(1), dim3(RS_TILE), 0, st, hist, ntiles, skip);
-        hipLaunchKernelGGL(k_rs_scatter, dim3(ntiles), dim3(RS_TILE), 0, st, kin[pass], vin[pass], kout[pass],
+        hipLaunchKernelGGL(k_rs_count, dim3(ntiles, rows), dim3(RS_TILE), 0, st, kin[pass], n, shift, hist, ntiles,
+                           skip);
+        hipLaunchKernelGGL(k_rs_scatter, dim3(ntiles, rows), dim3(RS_TILE), 0, st, kin[pass], vin[pass], kout[pass],
                            vout[pass], n, shift, hist, ntiles, skip);
     }
     return (int)hipGetLastError();
 }
 
-extern "C" int l98k_smp_topp_dist(const float *probs, int n, const uint32_t *skeys, const int *svals,
-                                  const int *n_cand, float topp, float *p_out, const int *skip, hipStream_t st) {
-    hipLaunchKernelGGL(k_smp_topp_dist, dim3(1), dim3(SMP_THREADS), 0, st, probs, n, skeys, svals, n_cand, topp,
-                       p_out, skip);
+extern "C" size_t l98k_smp_topp_tmp_bytes(int rows) { return sizeof(TopP) * (size_t)rows; }
+
+extern "C" int l98k_smp_topp_dist(const float *probs, int n, int rows, const uint32_t *skeys, const int *svals,
+                                  const int *n_cand, float topp, void *tmp, float *p_out, const int *skip,
+                                  hipStream_t st) {
+    if (n < 1 || rows < 1 || !tmp) return -1;
+    TopP *t = reinterpret_cast<TopP *>(tmp);
+    hipLaunchKernelGGL(k_smp_topp_find, dim3(rows), dim3(SMP_THREADS), 0, st, probs, n, skeys, n_cand, topp, t, skip);
+    hipLaunchKernelGGL(k_smp_topp_fill, dim3((n + TOPP_TILE - 1) / TOPP_TILE, rows), dim3(TOPP_TILE), 0, st, n, skeys,
+                       svals, t, p_out, skip);
     return (int)hipGetLastError();
 }
 
