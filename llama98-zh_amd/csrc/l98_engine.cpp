@@ -1390,26 +1390,12 @@ struct DWide {
     // pinned memory and copied with one transfer (sized on demand)
     char *ctl_host = nullptr, *ctl_dev = nullptr;
     int ctl_cap = 0;
-    // the later parts of a split prefill chunk (see batch_capture_dev): each
-    // its own scratch and stream, and per part one event per layer plus two
-    std::vector<DWide *> peer;
-    std::vector<hipStream_t> pst;
-    std::vector<hipEvent_t> ev;
 };
 
 namespace {
 
 #define WIDE_MAX 512          // rows of one wide forward
 #define WIDE_MIN 16           // prefills shorter than this take the chunked path
-#define WIDE_SPLIT 64         // wide prefill chunks of at least this many rows run in parts
-#define WIDE_PARTS 3          // parts of a split chunk, each on its own stream (measured: 2 parts
-                              // 10.1 ms, 3 parts 9.7 ms, 4 parts 15.0 ms for a 512-row prefill; four
-                              // streams oversubscribe the process's four hardware queues)
-// Each part of a split chunk must exceed MAX_CHUNK rows: a part's rows run as
-// prefill items (wide_forward refuses a split part of MAX_CHUNK rows or
-// fewer), and the split is taken only when the last part also exceeds it.
-static_assert(((WIDE_SPLIT / WIDE_PARTS + MAX_CHUNK - 1) & ~(MAX_CHUNK - 1)) > MAX_CHUNK,
-              "the parts of the smallest split chunk must exceed MAX_CHUNK rows");
 
 // nullptr (the callers take the chunked path) for a SubLN model, whose
 // per-projection norms this many-row forward does not carry, and for a
@@ -1486,44 +1472,8 @@ DWide *wide_get(const DModel *cm) {
     return m->wide;
 }
 
-// The parts of a split prefill chunk: WIDE_PARTS - 1 peer scratches and
-// streams (default priority) and WIDE_PARTS x (n_layers + 2) events; false
-// when any of it cannot be made.
-bool wide_parts(DModel *m, DWide *w) {
-    if (!w->peer.empty()) return true;
-    std::vector<DWide *> peer;
-    std::vector<hipStream_t> pst;
-    std::vector<hipEvent_t> ev((size_t)WIDE_PARTS * (m->c.n_layers + 2), nullptr);
-    bool ok = true;
-    for (int p = 1; p < WIDE_PARTS && ok; p++) {
-        DWide *q = wide_alloc(m);
-        hipStream_t sq = nullptr;
-        ok = q && hipStreamCreateWithFlags(&sq, hipStreamNonBlocking) == hipSuccess;
-        if (q) peer.push_back(q);
-        if (sq) pst.push_back(sq);
-    }
-    for (auto &e : ev) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
-    if (!ok) {
-        for (auto &e : ev)
-            if (e) (void)hipEventDestroy(e);
-        for (auto sq : pst) (void)hipStreamDestroy(sq);
-        for (auto q : peer) wide_release(q);
-        return false;
-    }
-    w->peer = peer;
-    w->pst = pst;
-    w->ev = ev;
-    return true;
-}
-
 void wide_free(DModel *m) {
-    DWide *w = m->wide;
-    if (!w) return;
-    for (auto sq : w->pst) (void)hipStreamSynchronize(sq);
-    for (auto &e : w->ev) (void)hipEventDestroy(e);
-    for (auto sq : w->pst) (void)hipStreamDestroy(sq);
-    for (auto q : w->peer) wide_release(q);
-    wide_release(w);
+    wide_release(m->wide);
     m->wide = nullptr;
 }
 
@@ -1580,17 +1530,12 @@ static void pair_long_short(std::vector<AttnItem> &ai, const std::vector<int> &l
 // launch goes on stream st; the sessions' control blocks must hold their
 // slot bases and positions (pos_scratch = the item's pos0) before.
 int wide_forward(const DModel *m, DWide *w, const WideItem *items, int n_items, int R, bool advance, float *capture,
-                 float *logits, hipStream_t st, int pos_base = 0, hipEvent_t *wait_ev = nullptr,
-                 hipEvent_t *rec_ev = nullptr, int l0 = 0, int l1 = -1) {
+                 float *logits, hipStream_t st) {
     const LZModelConfig &c = m->c;
     const int d = c.hidden_size, E = c.num_experts, topk = c.num_experts_per_token;
     const int lat = c.moe_latent_dim, inter = c.moe_intermediate_size, sw = c.moe_shared_width;
     const float eps = c.rms_norm_eps;
-    if (l1 < 0) l1 = c.n_layers;
-    if (R < 1 || R > w->cap || n_items < 1 || n_items > w->cap || l0 < 0 || l0 >= l1 || l1 > c.n_layers) return 1;
-    // Layers [l0, l1) only (a split prefill enqueues its parts layer by layer,
-    // in turn): the tables, the attention scratch and the embedding come with
-    // layer 0, the final norm with the last layer.
+    if (R < 1 || R > w->cap || n_items < 1 || n_items > w->cap) return 1;
     // the sessions' tables for the item launches
     // Attention runs as one item launch per kernel: over the sessions'
     // verify rows, or over one session's prefill rows cut into MAX_CHUNK-row
@@ -1598,7 +1543,6 @@ int wide_forward(const DModel *m, DWide *w, const WideItem *items, int n_items, 
     // launch), else chunk by chunk.
     bool attn_items = n_items > 1;
     const bool prefill_items = n_items == 1 && items[0].n > MAX_CHUNK && !advance;
-    if ((pos_base || wait_ev || rec_ev) && !prefill_items) return 1;   // only a prefill chunk is split
     int n_attn = n_items;
     int max_len = 1, max_rows = 1;          // the attention items' longest row span and most rows
     int kda_max_n = 1;                      // the KDA items' most rows
@@ -1615,11 +1559,12 @@ int wide_forward(const DModel *m, DWide *w, const WideItem *items, int n_items, 
             ki[i] = KdaItem{s->kda, s->conv, &s->ctl->slot_base, s->kda_slot, s->conv_slot, I.row0, I.n, s->depth, 0};
             kda_max_n = I.n > kda_max_n ? I.n : kda_max_n;
             if (prefill_items) {
-                for (int c0 = 0; c0 < I.n; c0 += MAX_CHUNK) {
-                    const int nr = I.n - c0 < MAX_CHUNK ? I.n - c0 : MAX_CHUNK;
+                const int ir = l98k_attn_item_rows(c.head_dim, I.pos0 + I.n);
+                for (int c0 = 0; c0 < I.n; c0 += ir) {
+                    const int nr = I.n - c0 < ir ? I.n - c0 : ir;
                     ai.push_back(AttnItem{s->kq, s->vq, s->ks, s->vs, &s->ctl->pos_scratch, I.row0 + c0, nr,
-                                          s->seq_len, pos_base + c0});
-                    alen.push_back(I.pos0 + pos_base + c0 + nr);
+                                          s->seq_len, c0});
+                    alen.push_back(I.pos0 + c0 + nr);
                 }
             } else {
                 ai.push_back(AttnItem{s->kq, s->vq, s->ks, s->vs, &s->ctl->pos_scratch, I.row0, I.n, s->seq_len, 0});
@@ -1632,13 +1577,12 @@ int wide_forward(const DModel *m, DWide *w, const WideItem *items, int n_items, 
             n_attn = (int)ai.size();
         }
         for (const AttnItem &x : ai) max_rows = x.n > max_rows ? x.n : max_rows;
-        if (l0 == 0) {
-            CK(hipMemcpyAsync(w->kitems, ki.data(), sizeof(KdaItem) * ki.size(), hipMemcpyHostToDevice, st));
-            CK(hipMemcpyAsync(w->aitems, ai.data(), sizeof(AttnItem) * ai.size(), hipMemcpyHostToDevice, st));
-        }
+        CK(hipMemcpyAsync(w->kitems, ki.data(), sizeof(KdaItem) * ki.size(), hipMemcpyHostToDevice, st));
+        CK(hipMemcpyAsync(w->aitems, ai.data(), sizeof(AttnItem) * ai.size(), hipMemcpyHostToDevice, st));
     }
     const size_t att_item = (size_t)MAX_CHUNK * c.n_heads * (size_t)((max_len + 3) & ~3);
-    if (l0 == 0 && attn_items && w->att_items_floats < att_item * n_attn) {
+    if (attn_items && l98k_attn_items_need_att(c.head_dim, max_len, max_rows, prefill_items ? 1 : 0) &&
+        w->att_items_floats < att_item * n_attn) {
         CK(hipStreamSynchronize(st));
         if (w->att_items) (void)hipFree(w->att_items);
         w->att_items = nullptr;
@@ -1646,10 +1590,10 @@ int wide_forward(const DModel *m, DWide *w, const WideItem *items, int n_items, 
         CK(hipMalloc((void **)&w->att_items, sizeof(float) * att_item * n_attn));
         w->att_items_floats = att_item * n_attn;
     }
-    if (l0 == 0) CK(l98k_embed(m->embed.q, m->embed.s, w->toks, d, m->embed.gs, R, w->x, st));
+    CK(l98k_embed(m->embed.q, m->embed.s, w->toks, d, m->embed.gs, R, w->x, st));
     // every layer leaves its two residual addends in up_out and sd_out
-    const float *ra = l0 ? w->up_out : nullptr, *rb = l0 ? w->sd_out : nullptr;
-    for (int l = l0; l < l1; l++) {
+    const float *ra = nullptr, *rb = nullptr;
+    for (int l = 0; l < c.n_layers; l++) {
         const DLayer &L = m->L[l];
         CK(l98k_rmsnorm(w->x, d, ra, rb, L.in_norm, d, eps, R, nullptr, 0, w->xq, w->xqs, st));
         if (L.type == 1) {
@@ -1680,14 +1624,11 @@ int wide_forward(const DModel *m, DWide *w, const WideItem *items, int n_items, 
                     const size_t off = (size_t)plane * s->seq_len * kvd;
                     p.kcache = s->kq + off; p.vcache = s->vq + off;
                     p.kscale = s->ks + off / 32; p.vscale = s->vs + off / 32;
-                    p.ctl_pos = &s->ctl->pos_scratch; p.pos_off = pos_base;
+                    p.ctl_pos = &s->ctl->pos_scratch; p.pos_off = 0;
                     CK(l98k_attn_prep(&p, I.n, st));
                 }
-                // (a split chunk's second half reads the first half's K and V rows)
-                if (wait_ev) CK(hipStreamWaitEvent(st, wait_ev[l], 0));
                 CK(l98k_attn_items(&a, w->aitems, n_attn, plane, max_len, max_rows, w->att_items, att_item,
                                    prefill_items ? 1 : 0, st));
-                if (rec_ev) CK(hipEventRecord(rec_ev[l], st));
             }
             for (int it = 0; it < n_items && !attn_items; it++) {
                 const WideItem &I = items[it];
@@ -1750,11 +1691,7 @@ int wide_forward(const DModel *m, DWide *w, const WideItem *items, int n_items, 
                 a.xq += r0 * value; a.xqs += r0 * (value / 32);
                 a.rec = w->kda_rec;
                 a.orow = w->kda_o;
-                // (a split chunk's second half starts from the state and conv
-                // history the first half leaves)
-                if (wait_ev) CK(hipStreamWaitEvent(st, wait_ev[l], 0));
                 CK(l98k_kda_split(&a, items[0].n, kd, c.conv_kernel, st));
-                if (rec_ev) CK(hipEventRecord(rec_ev[l], st));
             } else {
                 CK(l98k_kda_items(&a, w->kitems, n_items, kda_max_n, (size_t)li * nv * kd * c.lin_v_head_dim,
                                   (size_t)li * c.lin_conv_dim * hist, kd, c.conv_kernel, st));
@@ -1784,7 +1721,6 @@ int wide_forward(const DModel *m, DWide *w, const WideItem *items, int n_items, 
         ra = w->up_out;
         rb = w->sd_out;
     }
-    if (l1 < c.n_layers) return 0;
     CK(l98k_rmsnorm(w->x, d, ra, rb, m->final_norm, d, eps, R, capture, d, logits ? w->xq : nullptr, w->xqs, st));
     if (logits) CK(mf(m->embed, w->xq, w->xqs, R, logits, c.vocab_size, st));
     return 0;
@@ -2036,50 +1972,23 @@ int batch_capture_dev(DState *d, LZRunState *s, const int *tokens, int n, int po
     CK(hipMemcpyAsync(d->tokbuf, tokens, sizeof(int) * (size_t)n, hipMemcpyHostToDevice, d->st));
     DWide *w = n >= WIDE_MIN ? wide_get(d->m) : nullptr;
     if (w) {
-        // wide chunks of up to WIDE_MAX rows: each one's positions start at
-        // pos_scratch, which the chunk's own control write moves along.  A
-        // chunk of at least WIDE_SPLIT rows runs as WIDE_PARTS parts, each on
-        // its own stream with its own scratch: part p's layer l waits, before
-        // its KDA recurrence or attention, for part p - 1's (the state, conv
-        // history and K/V rows of the rows before it), so each part's serial
-        // recurrence overlaps the other parts' remaining work.
-        DModel *dm = const_cast<DModel *>(d->m);
+        // wide chunks of up to WIDE_MAX rows on the session's stream: each one's
+        // positions start at pos_scratch, which the chunk's own control write
+        // moves along.  (Parts of a chunk on three streams, each layer waiting
+        // for the part before, so that one part's recurrence ran beside the
+        // others' GEMMs, paid while the recurrence was three times as long and
+        // the GEMMs had 16-row tiles: the many small launches and the waits
+        // between streams now cost what they hide.  511 rows of the 24-layer
+        // model take 7.8 ms on one stream, 6.0 to 10 ms on two or three
+        // depending on which hardware queues a process's streams share; 99
+        // rows 4.1 and 6.0 ms.)
         for (int done = 0; done < n;) {
             const int k = n - done < w->cap ? n - done : w->cap;
             h.pos_scratch = pos0 + done;
             CK(ctl_put(d, h));
-            const int kp = ((k + WIDE_PARTS - 1) / WIDE_PARTS + MAX_CHUNK - 1) & ~(MAX_CHUNK - 1);
-            if (k >= WIDE_SPLIT && k - (WIDE_PARTS - 1) * kp > MAX_CHUNK && wide_parts(dm, w)) {
-                const int L = c.n_layers, E = L + 2;
-                hipEvent_t *ev = w->ev.data();             // part p: ev[p * E + l], start E - 2, end E - 1
-                CK(hipEventRecord(ev[E - 2], d->st));      // the other streams start after the control write
-                // the parts' layers are enqueued in turn (layer 0 of every
-                // part, then layer 1, ...), so every stream has work from the
-                // start and each wait follows the record it waits for
-                for (int l = 0; l < L; l++) {
-                    for (int p = 0; p < WIDE_PARTS; p++) {
-                        DWide *wp = p ? w->peer[p - 1] : w;
-                        hipStream_t sp = p ? w->pst[p - 1] : d->st;
-                        const int r0 = p * kp, kr = p + 1 < WIDE_PARTS ? kp : k - r0;
-                        if (l == 0) {
-                            if (p) CK(hipStreamWaitEvent(sp, ev[E - 2], 0));
-                            CK(hipMemcpyAsync(wp->toks, d->tokbuf + done + r0, sizeof(int) * (size_t)kr,
-                                              hipMemcpyDeviceToDevice, sp));
-                        }
-                        const WideItem item{d, 0, kr, pos0 + done + r0};
-                        CK(wide_forward(d->m, wp, &item, 1, kr, false,
-                                        d->hcap + (size_t)(done + r0) * c.hidden_size, nullptr, sp, r0,
-                                        p ? ev + (size_t)(p - 1) * E : nullptr,
-                                        p + 1 < WIDE_PARTS ? ev + (size_t)p * E : nullptr, l, l + 1));
-                        if (p && l == L - 1) CK(hipEventRecord(ev[(size_t)p * E + E - 1], sp));
-                    }
-                }
-                for (int p = 1; p < WIDE_PARTS; p++) CK(hipStreamWaitEvent(d->st, ev[(size_t)p * E + E - 1], 0));
-            } else {
-                CK(hipMemcpyAsync(w->toks, d->tokbuf + done, sizeof(int) * (size_t)k, hipMemcpyDeviceToDevice, d->st));
-                const WideItem item{d, 0, k, pos0 + done};
-                CK(wide_forward(d->m, w, &item, 1, k, false, d->hcap + (size_t)done * c.hidden_size, nullptr, d->st));
-            }
+            CK(hipMemcpyAsync(w->toks, d->tokbuf + done, sizeof(int) * (size_t)k, hipMemcpyDeviceToDevice, d->st));
+            const WideItem item{d, 0, k, pos0 + done};
+            CK(wide_forward(d->m, w, &item, 1, k, false, d->hcap + (size_t)done * c.hidden_size, nullptr, d->st));
             done += k;
             lz_debug_n_chunks++;
         }

@@ -1,6 +1,8 @@
 // Attention kernels against the Q8 KV cache
 // (bit-exact restatement of the reference float-oracle path; see
 // l98_devmath.h for the numeric contract).
+#include <type_traits>
+
 #include "l98_devmath.h"
 
 // ------------------------------------------------------------ attention ---
@@ -1010,6 +1012,22 @@ struct ArPlan {
                   "chunk staging layout");
 };
 
+// Lane I of each 16-lane row, on every lane of the row (row_newbcast:I): an
+// operand modifier of the multiply that takes it, so a value that 64 lanes
+// share costs an instruction neither to fetch nor to spread.
+template <int I>
+__device__ __forceinline__ float ar_row(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + I, 0xF, 0xF, true));
+}
+// f(integral constant I) for I = 0 .. N - 1
+template <int N, int I = 0, class F>
+__device__ __forceinline__ void ar_each(F &&f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>());
+        ar_each<N, I + 1>(f);
+    }
+}
+
 template <int HD, int WPT>
 __global__ __launch_bounds__(AR_THREADS) void k_attn_rows(AttnArgs b, const AttnItem *__restrict__ items,
                                                           int plane, int lp) {
@@ -1128,6 +1146,15 @@ __global__ __launch_bounds__(AR_THREADS) void k_attn_rows(AttnArgs b, const Attn
         float *s_part = s_ks + SCH * NB;                                               // [TPB][NB][SCH]
         const float scale = a.attn_scale;
         const int g = wave / WPG, pl = (wave - g * WPG) * 64 + lane;
+        // the group's 32 elements of every token's q head, 16 to a lane row:
+        // the products take them by row broadcast (read from LDS in the loop,
+        // 16 bytes for four products, they took twice the products' time)
+        float q0[TPB], q1[TPB];
+#pragma unroll
+        for (int j = 0; j < TPB; j++) {
+            q0[j] = s_q[j][g * 32 + (lane & 15)];
+            q1[j] = s_q[j][g * 32 + 16 + (lane & 15)];
+        }
         for (int c0 = 0; c0 < Lmax; c0 += SCH) {
             const int nc = imin(SCH, Lmax - c0);
 #pragma unroll
@@ -1147,13 +1174,23 @@ __global__ __launch_bounds__(AR_THREADS) void k_attn_rows(AttnArgs b, const Attn
                 float acc[TPB];
 #pragma unroll
                 for (int j = 0; j < TPB; j++) acc[j] = 0.0f;
-#pragma unroll
-                for (int e = 0; e < 32; e++) {
-                    const int w = e < 16 ? k0[e >> 2] : k1[(e - 16) >> 2];
+                ar_each<32>([&](auto ec) {
+                    constexpr int e = decltype(ec)::value;
+                    const int w = e < 16 ? k0[(e & 15) >> 2] : k1[(e & 15) >> 2];
                     const float kf = (float)(int8_t)((w >> (8 * (e & 3))) & 0xFF);
+                    float t4[TPB];
 #pragma unroll
-                    for (int j = 0; j < TPB; j++) acc[j] += s_q[j][g * 32 + e] * kf;
-                }
+                    for (int j = 0; j < TPB; j++) t4[j] = ar_row<e & 15>(e < 16 ? q0[j] : q1[j]) * kf;
+                    // (the products in registers of their own: a broadcast product
+                    // into the register of the one before waits a slot)
+                    if constexpr (TPB == 8)
+                        asm("" : "+v"(t4[0]), "+v"(t4[1]), "+v"(t4[2]), "+v"(t4[3]), "+v"(t4[TPB - 4]), "+v"(t4[TPB - 3]),
+                                 "+v"(t4[TPB - 2]), "+v"(t4[TPB - 1]));
+                    else
+                        asm("" : "+v"(t4[0]), "+v"(t4[1]), "+v"(t4[2]), "+v"(t4[3]));
+#pragma unroll
+                    for (int j = 0; j < TPB; j++) acc[j] += t4[j];
+                });
                 const float ks = s_ks[pc * NB + g];
 #pragma unroll
                 for (int j = 0; j < TPB; j++) s_part[(j * NB + g) * SCH + pl] = acc[j] * ks;
@@ -1226,69 +1263,69 @@ __global__ __launch_bounds__(AR_THREADS) void k_attn_rows(AttnArgs b, const Attn
             const int pa = __builtin_amdgcn_readfirstlane(imax(0, imin(nc, La - c0)));
             const int pb = __builtin_amdgcn_readfirstlane(imax(0, imin(nc, Lb - c0)));
             if (vwork && pb > 0) {
-                const int pa4 = pa & ~3;
                 const float *a0 = s_a + (size_t)t0 * lp + c0, *a1 = a0 + lp;
                 const float *vsr = s_vst + (dv >> 5) * VCH, *vc = s_vf + dv;
-                // four positions a step, in two register sets: the next
-                // step's reads are issued before this step's products (past
-                // the end they read the last step again); the scheduling
-                // barrier keeps them above the products, and the empty asm
-                // after the products takes their registers, so they neither
-                // wait before the products nor fold into the next step
-#define AR_V_READ(S, q)                                                                     \
-    S##x0 = *reinterpret_cast<const v4f_a *>(a0 + (q));                                     \
-    S##x1 = *reinterpret_cast<const v4f_a *>(a1 + (q));                                     \
-    S##s = *reinterpret_cast<const v4f_a *>(vsr + (q));                                     \
-    S##v0 = vc[(q) * VS];                                                                   \
-    S##v1 = vc[((q) + 1) * VS];                                                             \
-    S##v2 = vc[((q) + 2) * VS];                                                             \
-    S##v3 = vc[((q) + 3) * VS]
-#define AR_V_STEP(S)                                                                        \
-    {                                                                                       \
-        const float q0 = S##x0[0] * S##v0 * S##s[0], q1 = S##x0[1] * S##v1 * S##s[1];       \
-        const float q2 = S##x0[2] * S##v2 * S##s[2], q3 = S##x0[3] * S##v3 * S##s[3];       \
-        const float r0 = S##x1[0] * S##v0 * S##s[0], r1 = S##x1[1] * S##v1 * S##s[1];       \
-        const float r2 = S##x1[2] * S##v2 * S##s[2], r3 = S##x1[3] * S##v3 * S##s[3];       \
-        o0 += q0;                                                                           \
-        o1 += r0;                                                                           \
-        o0 += q1;                                                                           \
-        o1 += r1;                                                                           \
-        o0 += q2;                                                                           \
-        o1 += r2;                                                                           \
-        o0 += q3;                                                                           \
-        o1 += r3;                                                                           \
-    }
-#define AR_V_HOLD(S)                                                                        \
-    asm volatile("" : "+v"(o0), "+v"(o1), "+v"(S##x0), "+v"(S##x1), "+v"(S##s), "+v"(S##v0), \
-                 "+v"(S##v1), "+v"(S##v2), "+v"(S##v3))
-                if (pa4 > 0) {
-                    v4f_a Ax0, Ax1, As, Bx0, Bx1, Bs;
-                    float Av0, Av1, Av2, Av3, Bv0, Bv1, Bv2, Bv3;
-                    AR_V_READ(A, 0);
-                    for (int p = 0;; p += 8) {
-                        AR_V_READ(B, imin(p + 4, pa4 - 4));
-                        __builtin_amdgcn_sched_barrier(0);
-                        AR_V_STEP(A);
-                        AR_V_HOLD(B);
-                        if (p + 4 >= pa4) break;
-                        AR_V_READ(A, imin(p + 8, pa4 - 4));
-                        __builtin_amdgcn_sched_barrier(0);
-                        AR_V_STEP(B);
-                        AR_V_HOLD(A);
-                        if (p + 8 >= pa4) break;
-                    }
-                }
-#undef AR_V_READ
-#undef AR_V_STEP
-#undef AR_V_HOLD
+                const int l16 = lane & 15;
+                // sixteen positions a step: the probabilities and scales of one
+                // read per lane, 16 to a lane row, taken by row broadcast (a
+                // row's lanes share a 32-group's scale); the values one read
+                // per position for two tokens.  With the probabilities and
+                // scales read by every lane for every position, LDS reads took
+                // 2.7 times the products' time.  The next step's reads are in
+                // flight during this one's products.
+                struct Step {
+                    float x0, x1, s, v[16];
+                };
+                auto rd = [&](Step &k, int p) {
+                    const int pc = imin(p + l16, pb - 1);          // past the end: not used
+                    k.x0 = a0[pc];
+                    k.x1 = a1[pc];
+                    k.s = vsr[p + l16];
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const int p = pa4 + j;
-                    if (p >= pb) break;
-                    const float v = vc[p * VS], s = vsr[p];
-                    if (p < pa) o0 += a0[p] * v * s;
-                    o1 += a1[p] * v * s;
+                    for (int i = 0; i < 16; i++) k.v[i] = vc[(p + i) * VS];
+                };
+                auto step = [&](const Step &k) {
+                    ar_each<8>([&](auto ic) {
+                        constexpr int i = 2 * decltype(ic)::value;
+                        float t0_ = ar_row<i>(k.x0) * k.v[i], t1_ = ar_row<i>(k.x1) * k.v[i];
+                        float u0_ = ar_row<i + 1>(k.x0) * k.v[i + 1], u1_ = ar_row<i + 1>(k.x1) * k.v[i + 1];
+                        asm("" : "+v"(t0_), "+v"(t1_), "+v"(u0_), "+v"(u1_));
+                        float m0 = ar_row<i>(k.s) * t0_, m1 = ar_row<i>(k.s) * t1_;
+                        float n0 = ar_row<i + 1>(k.s) * u0_, n1 = ar_row<i + 1>(k.s) * u1_;
+                        asm("" : "+v"(m0), "+v"(m1), "+v"(n0), "+v"(n1));
+                        o0 += m0;
+                        o1 += m1;
+                        o0 += n0;
+                        o1 += n1;
+                    });
+                };
+                const int nf = pa >> 4;                            // whole steps (of both tokens)
+                Step A, B;
+                rd(A, 0);
+                int k = 0;
+                for (; k + 1 < nf; k += 2) {
+                    rd(B, 16 * (k + 1));
+                    __builtin_amdgcn_sched_barrier(0);
+                    step(A);
+                    if (16 * (k + 2) < VCH) rd(A, 16 * (k + 2));
+                    __builtin_amdgcn_sched_barrier(0);
+                    step(B);
                 }
+                if (k < nf) {
+                    if (16 * (k + 1) < VCH) rd(B, 16 * (k + 1));
+                    __builtin_amdgcn_sched_barrier(0);
+                    step(A);
+                    A = B;
+                    k++;
+                }
+                // the last positions: ra of t0, rb of t0 + 1
+                const int ra = pa - 16 * k, rb = pb - 16 * k;
+                if (rb > 0)
+                    ar_each<16>([&](auto ic) {
+                        constexpr int i = decltype(ic)::value;
+                        if (i < ra) o0 += ar_row<i>(A.s) * (ar_row<i>(A.x0) * A.v[i]);
+                        if (i < rb) o1 += ar_row<i>(A.s) * (ar_row<i>(A.x1) * A.v[i]);
+                    });
             }
         }
     }
@@ -1452,15 +1489,41 @@ static void av_allow_lds() {
 // plane bases and position; base carries the layer's weights and the row
 // buffers at row 0.  max_len: the longest item's last position + 1; att:
 // n_items scratch blocks of att_item floats.
+// The LDS of k_attn_rows for items of at most nmax rows and max_len positions
+// (two waves per token, four tokens, when every item has at most half a chunk
+// of rows), or 0 when it does not take them.
+static int ar_wpt(int nmax) { return nmax <= MAX_CHUNK / 2 ? 2 : 1; }
+static size_t ar_lds_bytes(int hd, int max_len, int nmax) {
+    if ((hd != 64 && hd != 128) || nmax < 1 || nmax > MAX_CHUNK) return 0;
+    const size_t lds = (size_t)(hd == 128 ? ArPlan<128>::STAGE : ArPlan<64>::STAGE) +
+                       (size_t)(MAX_CHUNK / ar_wpt(nmax)) * ((max_len + 3) & ~3) * sizeof(float);
+    return lds <= (size_t)(lds_limit() - AR_STATIC_MARGIN) ? lds : 0;
+}
+// Rows per item that a prefill's rows are best cut into: MAX_CHUNK, or half of
+// it past the contexts whose eight score rows fit the LDS (about 3,600
+// positions for 128-wide heads): at 4,001 positions k_attn_rows takes 0.9 ms
+// with four rows per item, k_attn_scores_items and k_attn_av_items 3.5 ms.
+extern "C" int l98k_attn_item_rows(int hd, int max_len) {
+    return !ar_lds_bytes(hd, max_len, MAX_CHUNK) && ar_lds_bytes(hd, max_len, MAX_CHUNK / 2) ? MAX_CHUNK / 2
+                                                                                            : MAX_CHUNK;
+}
+static bool avr_fits(int hd, int max_len) { return hd == AVR_HD && max_len <= AVR_L; }
+// 1 when l98k_attn_items keeps these items' score rows in att.
+extern "C" int l98k_attn_items_need_att(int hd, int max_len, int nmax, int kv_cached) {
+    return !(avr_fits(hd, max_len) ? kv_cached != 0 : ar_lds_bytes(hd, max_len, nmax) != 0);
+}
+
 extern "C" int l98k_attn_items(const AttnArgs *a, const AttnItem *items, int n_items, int plane, int max_len,
                                int nmax, float *att, size_t att_item, int kv_cached, hipStream_t st) {
     if (a->nkv < 1 || a->nh % a->nkv || (a->hd & 31) || 256 % a->hd || a->hd > ATT_MAX_HD || a->rot > a->hd ||
-        (a->rot & 1) || n_items < 1 || max_len < 1 || !a->oq || !a->oqs || !att || a->kv_only)
+        (a->rot & 1) || n_items < 1 || max_len < 1 || !a->oq || !a->oqs || a->kv_only)
         return -1;
     if (a->nh / a->nkv + MAX_CHUNK > ATT_MAX_VEC) return -1;
     const int att_stride = (max_len + 3) & ~3;
-    if ((size_t)MAX_CHUNK * a->nh * att_stride > att_item) return -1;
-    const bool rows = a->hd == AVR_HD && max_len <= AVR_L;
+    if (l98k_attn_items_need_att(a->hd, max_len, nmax, kv_cached) &&
+        (!att || (size_t)MAX_CHUNK * a->nh * att_stride > att_item))
+        return -1;
+    const bool rows = avr_fits(a->hd, max_len);
     if (rows && kv_cached) {
         // every row's K is in the cache: the value-sum blocks take their scores
         hipLaunchKernelGGL(k_attn_av_rows, dim3(a->nh, n_items), dim3(512), 0, st, *a, items, plane, att, att_stride,
@@ -1471,11 +1534,9 @@ extern "C" int l98k_attn_items(const AttnArgs *a, const AttnItem *items, int n_i
     // rows into the caches first (unless they are there), then one block per
     // (q head, item) with the score rows in LDS, two waves per token when
     // every item has at most half a chunk of rows
-    const int wpt = nmax <= MAX_CHUNK / 2 ? 2 : 1;
-    const size_t ar_lds = (size_t)(a->hd == 128 ? ArPlan<128>::STAGE : ArPlan<64>::STAGE) +
-                          (size_t)(MAX_CHUNK / wpt) * att_stride * sizeof(float);
-    if (!rows && (a->hd == 64 || a->hd == 128) && nmax >= 1 && nmax <= MAX_CHUNK &&
-        ar_lds <= (size_t)(lds_limit() - AR_STATIC_MARGIN)) {
+    const int wpt = ar_wpt(nmax);
+    const size_t ar_lds = ar_lds_bytes(a->hd, max_len, nmax);
+    if (!rows && ar_lds) {
         if (!kv_cached) {
             hipLaunchKernelGGL(k_attn_prep_items, dim3(2 * a->nkv, MAX_CHUNK, n_items), dim3(64), 0, st, *a, items,
                                plane);

@@ -137,8 +137,13 @@ int l98k_attn_prep(const AttnArgs *a, int nt, hipStream_t st);
 int l98k_attn_t1(const float *qg, int qg_dim, const float *vp, int kv_dim, int nh, int nkv, int hd, int q_dim,
                  int rows, int8_t *vc0, float *vs0, float *out, int8_t *oq, float *oqs, hipStream_t st);
 // Attention of several sessions' rows in one launch per kernel (items in
-// device memory); att: n_items blocks of att_item floats.  kv_cached: every
-// row's K and V are already in the cache (a prefill after its K/V launch).
+// device memory, of at most nmax rows); att: n_items blocks of att_item
+// floats, where l98k_attn_items_need_att says that the score rows go through
+// it.  kv_cached: every row's K and V are already in the cache (a prefill after
+// its K/V launch).  l98k_attn_item_rows: the rows per item to cut a prefill
+// into.
+int l98k_attn_item_rows(int hd, int max_len);
+int l98k_attn_items_need_att(int hd, int max_len, int nmax, int kv_cached);
 int l98k_attn_prep_items(const AttnArgs *a, const AttnItem *items, int n_items, int plane, hipStream_t st);
 int l98k_attn_items(const AttnArgs *a, const AttnItem *items, int n_items, int plane, int max_len, int nmax,
                     float *att, size_t att_item, int kv_cached, hipStream_t st);
