@@ -1581,7 +1581,7 @@ int wide_forward(const DModel *m, DWide *w, const WideItem *items, int n_items, 
         CK(hipMemcpyAsync(w->aitems, ai.data(), sizeof(AttnItem) * ai.size(), hipMemcpyHostToDevice, st));
     }
     const size_t att_item = (size_t)MAX_CHUNK * c.n_heads * (size_t)((max_len + 3) & ~3);
-    if (attn_items && l98k_attn_items_need_att(c.head_dim, max_len, max_rows, prefill_items ? 1 : 0) &&
+    if (attn_items && l98k_attn_items_need_att(c.head_dim, max_len, max_rows) &&
         w->att_items_floats < att_item * n_attn) {
         CK(hipStreamSynchronize(st));
         if (w->att_items) (void)hipFree(w->att_items);
@@ -3419,7 +3419,7 @@ int greedy_rounds_batched(const LZModel *mm, LZRunState **states, int n_seq, int
         w->logits_rows = R;
     }
     const size_t att_item = (size_t)MAX_CHUNK * c.n_heads * (size_t)((max_len + 3) & ~3);
-    if (w->att_items_floats < att_item * n_seq) {
+    if (l98k_attn_items_need_att(c.head_dim, max_len, 1) && w->att_items_floats < att_item * n_seq) {
         if (w->att_items) (void)hipFree(w->att_items);
         w->att_items = nullptr;
         w->att_items_floats = 0;

@@ -824,148 +824,6 @@ __global__ __launch_bounds__(AG_THREADS) void k_attn_avg(AttnArgs a, const float
     }
 }
 
-// k_attn_av_rows: the softmax and value sums of an item launch whose rows
-// all lie below position 512, for 64-wide heads: one block per (q head,
-// item), wave t = the item's token t, lane = output element d.  The item's
-// V rows are staged once for its eight tokens, transposed ([d][position],
-// and the scales [group][position]), so a lane reads four positions' bytes
-// in one access; each wave takes its token's softmax (max, exp, the exact
-// wave sum of the serial loop, scale), then lane d adds (a[p] * v[p][d]) *
-// vs[p][d/32] over positions p = 0 .. pos in order - the arithmetic of
-// attn_av_body, per token.  Then the gate and the per-32 quantization.
-#define AVR_L 512
-#define AVR_HD 64
-__global__ __launch_bounds__(512) void k_attn_av_rows(AttnArgs b, const AttnItem *__restrict__ items, int plane,
-                                                      const float *__restrict__ att, int att_stride, size_t att_item,
-                                                      int own_scores) {
-    EXP_TAB_LOAD(tab);
-    __shared__ __align__(16) int8_t s_vt[AVR_HD][AVR_L];          // V transposed
-    __shared__ __align__(16) float s_vst[AVR_HD / 32][AVR_L];     // its scales, transposed
-    __shared__ __align__(16) float s_a[MAX_CHUNK][AVR_L];         // scores, then probabilities
-    __shared__ __align__(16) float s_e[MAX_CHUNK][64 * (8 + 4)];  // exps in the exact sum's layout (8 per lane)
-    __shared__ PsRec s_rec[MAX_CHUNK][128];
-    __shared__ __align__(16) float s_q[MAX_CHUNK][AVR_HD];        // own_scores: the prepared q heads
-    const int h = blockIdx.x, item = blockIdx.y;
-    const AttnItem it = items[item];
-    const AttnArgs a = attn_item_args(b, it, plane);
-    const float *arows = att + (size_t)item * att_item;
-    const int tid = threadIdx.x, t = tid >> 6, lane = tid & 63;
-    const int kv_mul = a.nh / a.nkv, kvh = h / kv_mul, nb = AVR_HD / 32;
-    const int pos0 = *a.ctl_pos + a.pos_off, n = it.n, Lmax = pos0 + n;
-    const bool live = t < n;
-    const int L = pos0 + imin(t, n - 1) + 1;
-    // stage: V rows [0, Lmax) of the kv head (4 int4 per row), their scales,
-    // and each wave's score row
-    for (int f = tid; f < Lmax * 4; f += 512) {
-        const int p = f >> 2, c = f & 3;
-        const int4 v4 = *reinterpret_cast<const int4 *>(a.vcache + (size_t)p * a.kv_dim + kvh * AVR_HD + 16 * c);
-        const int w4[4] = {v4.x, v4.y, v4.z, v4.w};
-#pragma unroll
-        for (int k = 0; k < 16; k++) s_vt[16 * c + k][p] = (int8_t)((w4[k >> 2] >> (8 * (k & 3))) & 0xFF);
-    }
-    for (int f = tid; f < Lmax * nb; f += 512) {
-        const int p = f / nb, g = f - p * nb;
-        s_vst[g][p] = a.vscale[(size_t)p * (a.kv_dim >> 5) + kvh * nb + g];
-    }
-    if (live && !own_scores)
-        for (int p = lane; p < L; p += 64) s_a[t][p] = arows[((size_t)t * a.nh + h) * att_stride + p];
-    if (live && own_scores) {
-        // every K row is in the cache: the wave prepares its token's q head
-        // (RMSNorm(1+w) with the serial sum, NeoX rotary) and computes the
-        // scores itself, as k_attn_scores_items does
-        const int pos_t = L - 1, half = a.rot >> 1;
-        const float x = a.qg[(size_t)t * a.qg_dim + (size_t)h * 2 * AVR_HD + lane];
-        s_e[t][lane] = x * x;
-        __builtin_amdgcn_s_waitcnt(0xC07F);           // lgkmcnt(0): the squares are in LDS
-        __builtin_amdgcn_wave_barrier();
-        const float inv = d_rsqrt(d_ss_over_n(serial_sum(s_e[t], AVR_HD), AVR_HD) + a.eps);
-        const float y = x * inv * (1.0f + a.q_norm[lane]);
-        const float yo = __shfl(y, lane < half ? lane + half : lane - half);     // the rotary partner
-        float r = y;
-        if (lane < half) {
-            const float c = a.rope_cs[((size_t)pos_t * half + lane) * 2], sn = a.rope_cs[((size_t)pos_t * half + lane) * 2 + 1];
-            r = y * c - yo * sn;
-        } else if (lane < 2 * half) {
-            const int i = lane - half;
-            const float c = a.rope_cs[((size_t)pos_t * half + i) * 2], sn = a.rope_cs[((size_t)pos_t * half + i) * 2 + 1];
-            r = y * c + yo * sn;
-        }
-        s_q[t][lane] = r;
-        __builtin_amdgcn_s_waitcnt(0xC07F);
-        __builtin_amdgcn_wave_barrier();
-        const float scale = a.attn_scale;
-        for (int p = lane; p < L; p += 64) {
-            const int8_t *kr = a.kcache + (size_t)p * a.kv_dim + kvh * AVR_HD;
-            const float *ks = a.kscale + (size_t)p * (a.kv_dim >> 5) + kvh * nb;
-            float sum = 0.0f;
-#pragma unroll
-            for (int dd = 0; dd < AVR_HD; dd += 32) {
-                const int4 k0 = *reinterpret_cast<const int4 *>(kr + dd);
-                const int4 k1 = *reinterpret_cast<const int4 *>(kr + dd + 16);
-                const int8_t *kb0 = reinterpret_cast<const int8_t *>(&k0);
-                const int8_t *kb1 = reinterpret_cast<const int8_t *>(&k1);
-                float acc = 0.0f;
-#pragma unroll
-                for (int e = 0; e < 16; e++) acc += s_q[t][dd + e] * (float)kb0[e];
-#pragma unroll
-                for (int e = 0; e < 16; e++) acc += s_q[t][dd + 16 + e] * (float)kb1[e];
-                sum += acc * ks[dd >> 5];
-            }
-            s_a[t][p] = sum * scale;
-        }
-    }
-    EXP_TAB_PUT(tab);
-    __syncthreads();
-    // softmax of the wave's token: max (order-preserving key), exp, the
-    // serial loop's sum, scale
-    if (live) {
-        uint32_t best = 0;
-        for (int p = lane; p < L; p += 64) best = umax(best, d_fkey(s_a[t][p]));
-        for (int o = 32; o > 0; o >>= 1) best = umax(best, (uint32_t)__shfl_xor((int)best, o));
-        const float mx = d_unkey(best);
-        for (int p = lane; p < L; p += 64) {
-            const float e = d_exp(s_a[t][p] - mx, tab);
-            s_a[t][p] = e;
-            s_e[t][(p >> 3) * 12 + (p & 7)] = e;
-        }
-        // positions L .. of the padded row read as 0 inside the exact sum
-        __builtin_amdgcn_s_waitcnt(0xC07F);           // lgkmcnt(0): the wave's exps are in LDS
-        __builtin_amdgcn_wave_barrier();
-        const float sum = wave_sum_nonneg<8>(s_e[t], L, s_rec[t]);
-        const float inv = (sum > 0.0f) ? 1.0f / sum : 0.0f;
-        for (int p = lane; p < L; p += 64) s_a[t][p] *= inv;
-    }
-    __syncthreads();
-    if (!live) return;
-    // value sum, four positions per step (the adds stay in position order)
-    const int d = lane, g = d >> 5;
-    float o = 0.0f;
-    const int L4 = L & ~3;
-    for (int p = 0; p < L4; p += 4) {
-        const float4 ap = *reinterpret_cast<const float4 *>(&s_a[t][p]);
-        const uint32_t vb = *reinterpret_cast<const uint32_t *>(&s_vt[d][p]);
-        const float4 vs = *reinterpret_cast<const float4 *>(&s_vst[g][p]);
-        const float p0 = ap.x * (float)(int8_t)(vb & 0xFF) * vs.x;
-        const float p1 = ap.y * (float)(int8_t)((vb >> 8) & 0xFF) * vs.y;
-        const float p2 = ap.z * (float)(int8_t)((vb >> 16) & 0xFF) * vs.z;
-        const float p3 = ap.w * (float)(int8_t)(vb >> 24) * vs.w;
-        o += p0;
-        o += p1;
-        o += p2;
-        o += p3;
-    }
-    for (int p = L4; p < L; p++) o += s_a[t][p] * (float)s_vt[d][p] * s_vst[g][p];
-    const float gate = a.qg[(size_t)t * a.qg_dim + (size_t)h * 2 * AVR_HD + AVR_HD + d];
-    o *= d_sigmoid(gate, tab);
-    const int col = h * AVR_HD + d;
-    if (a.out) a.out[(size_t)t * a.q_dim + col] = o;
-    int8_t q;
-    float sg;
-    d_quant_group32(o, &q, &sg);
-    a.oq[(size_t)t * a.q_dim + col] = q;
-    if ((d & 31) == 0) a.oqs[(size_t)t * (a.q_dim >> 5) + (col >> 5)] = sg;
-}
-
 // k_attn_rows<HD, WPT>: the softmax and value sums of an item launch whose
 // K and V rows are all in the cache, 64- or 128-wide heads, positions up to
 // what the block's LDS holds (the launch checks): one block of 8 waves per
@@ -984,9 +842,18 @@ __global__ __launch_bounds__(512) void k_attn_av_rows(AttnArgs b, const AttnItem
 //   4. value sums, chunk by chunk of VCH = 8192 / HD V rows staged once as
 //      fp32 (row-major, scales [group][position]): a lane takes one element
 //      d of two consecutive tokens and adds (a[p] * v[p][d]) * vs[p][d/32]
-//      to each token's sum over the positions in order, four per step (one
-//      read of v for both; the LDS reads, not the VALU, bound this phase);
+//      to each token's sum over the positions in order, sixteen per step
+//      (one read of v for both);
 //   5. the sigmoid output gate and the per-32 quantization.
+// What several lanes share (q elements, probabilities, scales) is held 16
+// values to a lane row and taken by row broadcast, an operand modifier: read
+// from LDS per product, 16 bytes for four, those reads took longer than the
+// products.  Measured per launch: 64-wide heads, 511 rows of one session 47 us
+// (120 in the kernel it replaced there, one lane per element over a transposed
+// V); 128-wide, 32 sessions of 4 rows at up to 2,048 positions 105 us (120
+// with the LDS reads); 500 rows at 3,500 positions 0.85 ms, one block of eight
+// waves per CU since its score rows fill the LDS, bound by the waits of two
+// waves per SIMD.
 // Every chunk's global loads are issued into registers before the previous
 // chunk is computed (the first K chunk's before step 1, the first V chunk's
 // with the last K chunk), and stored to LDS after it.
@@ -1507,11 +1374,8 @@ extern "C" int l98k_attn_item_rows(int hd, int max_len) {
     return !ar_lds_bytes(hd, max_len, MAX_CHUNK) && ar_lds_bytes(hd, max_len, MAX_CHUNK / 2) ? MAX_CHUNK / 2
                                                                                             : MAX_CHUNK;
 }
-static bool avr_fits(int hd, int max_len) { return hd == AVR_HD && max_len <= AVR_L; }
 // 1 when l98k_attn_items keeps these items' score rows in att.
-extern "C" int l98k_attn_items_need_att(int hd, int max_len, int nmax, int kv_cached) {
-    return !(avr_fits(hd, max_len) ? kv_cached != 0 : ar_lds_bytes(hd, max_len, nmax) != 0);
-}
+extern "C" int l98k_attn_items_need_att(int hd, int max_len, int nmax) { return ar_lds_bytes(hd, max_len, nmax) == 0; }
 
 extern "C" int l98k_attn_items(const AttnArgs *a, const AttnItem *items, int n_items, int plane, int max_len,
                                int nmax, float *att, size_t att_item, int kv_cached, hipStream_t st) {
@@ -1520,23 +1384,16 @@ extern "C" int l98k_attn_items(const AttnArgs *a, const AttnItem *items, int n_i
         return -1;
     if (a->nh / a->nkv + MAX_CHUNK > ATT_MAX_VEC) return -1;
     const int att_stride = (max_len + 3) & ~3;
-    if (l98k_attn_items_need_att(a->hd, max_len, nmax, kv_cached) &&
+    if (l98k_attn_items_need_att(a->hd, max_len, nmax) &&
         (!att || (size_t)MAX_CHUNK * a->nh * att_stride > att_item))
         return -1;
-    const bool rows = avr_fits(a->hd, max_len);
-    if (rows && kv_cached) {
-        // every row's K is in the cache: the value-sum blocks take their scores
-        hipLaunchKernelGGL(k_attn_av_rows, dim3(a->nh, n_items), dim3(512), 0, st, *a, items, plane, att, att_stride,
-                           att_item, 1);
-        return (int)hipGetLastError();
-    }
-    // 64- or 128-wide heads past the rows kernel's reach: the new K and V
-    // rows into the caches first (unless they are there), then one block per
-    // (q head, item) with the score rows in LDS, two waves per token when
-    // every item has at most half a chunk of rows
+    // 64- or 128-wide heads whose score rows fit the LDS: the new K and V rows
+    // into the caches first (unless they are there), then one block per (q
+    // head, item), two waves per token when every item has at most half a
+    // chunk of rows
     const int wpt = ar_wpt(nmax);
     const size_t ar_lds = ar_lds_bytes(a->hd, max_len, nmax);
-    if (!rows && ar_lds) {
+    if (ar_lds) {
         if (!kv_cached) {
             hipLaunchKernelGGL(k_attn_prep_items, dim3(2 * a->nkv, MAX_CHUNK, n_items), dim3(64), 0, st, *a, items,
                                plane);
@@ -1572,11 +1429,6 @@ extern "C" int l98k_attn_items(const AttnArgs *a, const AttnItem *items, int n_i
                        plane, att, att_stride, att_item);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return (int)e;
-    if (rows) {
-        hipLaunchKernelGGL(k_attn_av_rows, dim3(a->nh, n_items), dim3(512), 0, st, *a, items, plane, att, att_stride,
-                           att_item, 0);
-        return (int)hipGetLastError();
-    }
     av_allow_lds();
     int ch = 0, sc = 0;
     size_t lds = 0;

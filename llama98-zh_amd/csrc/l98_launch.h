@@ -143,7 +143,7 @@ int l98k_attn_t1(const float *qg, int qg_dim, const float *vp, int kv_dim, int n
 // its K/V launch).  l98k_attn_item_rows: the rows per item to cut a prefill
 // into.
 int l98k_attn_item_rows(int hd, int max_len);
-int l98k_attn_items_need_att(int hd, int max_len, int nmax, int kv_cached);
+int l98k_attn_items_need_att(int hd, int max_len, int nmax);
 int l98k_attn_prep_items(const AttnArgs *a, const AttnItem *items, int n_items, int plane, hipStream_t st);
 int l98k_attn_items(const AttnArgs *a, const AttnItem *items, int n_items, int plane, int max_len, int nmax,
                     float *att, size_t att_item, int kv_cached, hipStream_t st);
