@@ -1708,9 +1708,9 @@ int wide_forward(const DModel *m, DWide *w, const WideItem *items, int n_items, 
         CK(l98k_moe_group(w->sel_idx, pairs, topk, E, w->ng, w->gexp, w->goff, w->gcnt, w->list, w->pair_token, st));
         const int maxg = pairs < E ? pairs : E;
         const int mean_cols = (pairs + maxg - 1) / maxg;
-        CK(l98k_mfma_gemm_grouped2(L.w1.q, L.w1.s, w->h1, L.w3.q, L.w3.s, w->h3, inter, lat, w->latq, w->latqs, w->ng,
-                                   maxg, w->gexp, w->goff, w->gcnt, w->list, w->pair_token, R, mean_cols, inter, st));
-        CK(l98k_wide_pro(1, w->h1, w->h3, inter, nullptr, nullptr, 0, inter, pairs, w->hq, w->hqs, st));
+        CK(l98k_mfma_gemm_pair(L.w1.q, L.w1.s, L.w3.q, L.w3.s, inter, lat, w->latq, w->latqs, w->ng, maxg, w->gexp,
+                               w->goff, w->gcnt, w->list, w->pair_token, R, mean_cols, pairs, w->h1, w->h3, w->hq,
+                               w->hqs, st));
         CK(l98k_mfma_gemm_grouped(L.w2.q, L.w2.s, lat, inter, w->hq, w->hqs, w->ng, maxg, w->gexp, w->goff, w->gcnt,
                                   w->list, nullptr, R, mean_cols, w->h2, lat, st));
         // the shared expert's SiLU-mul rows and the routed experts' combine, one launch

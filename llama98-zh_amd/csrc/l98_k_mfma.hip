@@ -23,6 +23,7 @@
 // of 16 weight rows x 64 token columns (a wave per 16 columns), K through
 // double-buffered LDS stages of MF_KC bytes (eight groups).
 #include "l98_devmath.h"
+#include "l98_launch.h"
 
 typedef int v4i_t __attribute__((ext_vector_type(4)));
 
@@ -309,12 +310,28 @@ __device__ __forceinline__ void mft_arrive() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
-template <int RT, int CT, int WR, int WC>
+//
+// PAIR (grouped only; RT = 2, WR = 2): the experts' w1 and w3 of the same 32
+// rows as one block's 64, a wave's two tiles being its 16 rows of each, so
+// that the lane holding w1's output holds w3's, and the block the whole
+// 32-element group of a column: it leaves silu(w1) * w3 quantized per 32
+// (mode 1 of k_wide_pro, the same arithmetic), and neither float matrix is
+// written.
+struct MfPair {
+    const int8_t *W3;                   // w3's bank and scales
+    const float *ws3;
+    int8_t *q;                          // [pairs][N] and [pairs][N / 32]
+    float *qs;
+};
+template <int RT, int CT, int WR, int WC, bool PAIR = false>
 __global__ __launch_bounds__(64 * WR * WC) void k_mfma_q8t(const int8_t *W0, const float *ws0, int N0, int K0,
                                                            size_t w_group_stride, const int8_t *X0, const float *Xs0,
                                                            int M, MfCols cols, float *out0, int out_stride0,
-                                                           MfJobs jobs) {
+                                                           MfJobs jobs, MfPair pair) {
     constexpr int TR = 16 * RT * WR, TC = 16 * CT * WC;   // the block's tile
+    constexpr int ORT = PAIR ? TR / 2 : TR;               // output rows of a tile
+    constexpr int AST = (PAIR ? 32 : 16) * MFT_KC;        // between a wave's tiles in LDS
+    static_assert(!PAIR || (RT == 2 && WR == 2 && CT == 1), "a pair tile: 32 rows of each bank");
     constexpr int NTHR = 64 * WR * WC, PW = TR * 8 / NTHR, PX = TC * 8 / NTHR, SL = TC / (WR * WC);
     static_assert(TR * 8 % NTHR == 0 && TC * 8 % NTHR == 0 && SL <= 64, "whole direct loads");
     constexpr int LPS = PW + PX + 1;                      // direct loads of a wave per stage
@@ -360,8 +377,8 @@ __global__ __launch_bounds__(64 * WR * WC) void k_mfma_q8t(const int8_t *W0, con
         bx -= jb.blk0;
     }
     int ncols = M, cbase = 0;
-    const int8_t *Wg = W;
-    const float *wsg = ws;
+    const int8_t *Wg = W, *Wg3 = PAIR ? pair.W3 : nullptr;
+    const float *wsg = ws, *wsg3 = PAIR ? pair.ws3 : nullptr;
     if (cols.list) {
         const int g = blockIdx.z;
         if (g >= *cols.ng) return;
@@ -370,17 +387,24 @@ __global__ __launch_bounds__(64 * WR * WC) void k_mfma_q8t(const int8_t *W0, con
         const int e = cols.gexp[g];
         Wg = W + (size_t)e * w_group_stride;
         wsg = ws + (size_t)e * N;
+        if constexpr (PAIR) {
+            Wg3 += (size_t)e * w_group_stride;
+            wsg3 += (size_t)e * N;
+        }
     }
-    const int n0 = bx * TR, nb = K >> 5, nst = K / MFT_KC;
+    float tabv = 0.0f;
+    if constexpr (PAIR) tabv = c_exp_tab[tid & 31];
+    const int n0 = bx * ORT, nb = K >> 5, nst = K / MFT_KC;
     // this thread's pieces of a stage: rows i NTHR / 8 + tid / 8, LDS place
     // tid % 8 (the row's bits 1..3 do not depend on i)
     const int prow = tid >> 3, gp = 16 * ((tid & 7) ^ ((prow >> 1) & 7));
     uint32_t wl[PW];
 #pragma unroll
-    for (int i = 0; i < PW; i++) wl[i] = (uint32_t)imin(n0 + NTHR / 8 * i + prow, N - 1) * (uint32_t)K + gp;
+    for (int i = 0; i < PW; i++)
+        wl[i] = (uint32_t)imin(n0 + (NTHR / 8 * i) % ORT + prow, N - 1) * (uint32_t)K + gp;
     // operand reads: lane l's 8 bytes 8 (l / 16) of group g of row l % 16
     const int r16 = lane & 15, q = lane >> 4;
-    const int wr0 = (wave % WR) * 16 * RT, wc0 = (wave / WR) * 16 * CT;
+    const int wr0 = (wave % WR) * 16 * (PAIR ? 1 : RT), wc0 = (wave / WR) * 16 * CT;
     int oa[4], ox[4];
 #pragma unroll
     for (int g = 0; g < 4; g++) {
@@ -405,11 +429,12 @@ __global__ __launch_bounds__(64 * WR * WC) void k_mfma_q8t(const int8_t *W0, con
         // group scales: lanes below SL of each wave, a column's four each
         const uint32_t xsl = (uint32_t)xrow(wave * SL + imin(lane, SL - 1)) * (uint32_t)nb * 4;
         auto issue = [&](int st, int b) {
-            const int8_t *wb = Wg + (size_t)st * MFT_KC, *xb = X + (size_t)st * MFT_KC;
+            const int8_t *wb = Wg + (size_t)st * MFT_KC, *wb3 = Wg3 + (size_t)st * MFT_KC;
+            const int8_t *xb = X + (size_t)st * MFT_KC;
             const int8_t *sb = reinterpret_cast<const int8_t *>(Xs) + (size_t)st * 16;
 #pragma unroll
             for (int i = 0; i < PW; i++)
-                __builtin_amdgcn_global_load_lds((mft_gptr)(wb + wl[i]),
+                __builtin_amdgcn_global_load_lds((mft_gptr)((NTHR / 8 * i < ORT ? wb : wb3) + wl[i]),
                                                  (mft_lptr)(&s_buf[b][(NTHR * i + 64 * wave) * 16]), 16, 0, 0);
 #pragma unroll
             for (int i = 0; i < PX; i++)
@@ -435,7 +460,7 @@ __global__ __launch_bounds__(64 * WR * WC) void k_mfma_q8t(const int8_t *W0, con
 #pragma unroll
             for (int g = 0; g < 4; g++) {
 #pragma unroll
-                for (int i = 0; i < RT; i++) ka[g][i] = *reinterpret_cast<const long *>(p + oa[g] + 16 * i * MFT_KC);
+                for (int i = 0; i < RT; i++) ka[g][i] = *reinterpret_cast<const long *>(p + oa[g] + i * AST);
 #pragma unroll
                 for (int j = 0; j < CT; j++) kx[g][j] = *reinterpret_cast<const long *>(p + ox[g] + 16 * j * MFT_KC);
                 if (g == 0)
@@ -487,6 +512,35 @@ __global__ __launch_bounds__(64 * WR * WC) void k_mfma_q8t(const int8_t *W0, con
             }
         }
         // lane l: rows 4 (l / 16) .. + 3 of a tile, column l % 16
+        if constexpr (PAIR) {
+            // (in the stage buffers, which every wave has read)
+            float *tab = reinterpret_cast<float *>(&s_buf[0][0]);
+            uint32_t *s_am = reinterpret_cast<uint32_t *>(&s_buf[0][128]);        // [WR][TC]
+            __syncthreads();
+            if (tid < 32) tab[tid] = tabv;
+            __syncthreads();
+            const int n = n0 + wr0 + 4 * q, col = wc0 + r16, cl = c0 + col;
+            float y[4];
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int nc = imin(n + v, N - 1);
+                const float h1 = 0.0f + f[0][0][v] * wsg[nc], h3 = 0.0f + f[1][0][v] * wsg3[nc];
+                y[v] = d_silu(h1, tab) * h3;
+            }
+            const float4 y4 = make_float4(y[0], y[1], y[2], y[3]);
+            uint32_t am = abs_bits4(y4);
+            am = umax(am, (uint32_t)__shfl_xor((int)am, 16));
+            am = umax(am, (uint32_t)__shfl_xor((int)am, 32));
+            if (q == 0) s_am[(wave % WR) * TC + col] = am;
+            __syncthreads();
+            float sg;
+            const uint32_t pk = quant4_amax(y4, f_from_u(umax(s_am[col], s_am[TC + col])), &sg);
+            if (cl < ncols) {
+                const size_t o = (size_t)cols.list[cbase + cl];
+                *reinterpret_cast<uint32_t *>(pair.q + o * N + n) = pk;
+                if (wave % WR == 0 && q == 0) pair.qs[o * (N >> 5) + (n0 >> 5)] = sg;
+            }
+        } else
 #pragma unroll
         for (int j = 0; j < CT; j++) {
             const int cl = c0 + wc0 + 16 * j + r16;
@@ -619,13 +673,13 @@ static void mft_launch(int t, dim3 grid, const int8_t *W, const float *ws, int N
                        const MfJobs &jobs, hipStream_t st) {
     if (t == MFT_32x16)
         hipLaunchKernelGGL((k_mfma_q8t<1, 1, 2, 1>), grid, dim3(128), 0, st, W, ws, N, K, w_group_stride, X, Xs, M, c,
-                           out, out_stride, jobs);
+                           out, out_stride, jobs, MfPair{});
     else if (t == MFT_32x32)
         hipLaunchKernelGGL((k_mfma_q8t<1, 1, 2, 2>), grid, dim3(256), 0, st, W, ws, N, K, w_group_stride, X, Xs, M, c,
-                           out, out_stride, jobs);
+                           out, out_stride, jobs, MfPair{});
     else
         hipLaunchKernelGGL((k_mfma_q8t<2, 1, 2, 2>), grid, dim3(256), 0, st, W, ws, N, K, w_group_stride, X, Xs, M, c,
-                           out, out_stride, jobs);
+                           out, out_stride, jobs, MfPair{});
 }
 // k_mfma_q8t takes offsets of 32 bits into a weight matrix and into the rows.
 static bool mft_ok(int N, int K, int rows) {
@@ -679,48 +733,59 @@ extern "C" int l98k_mfma_gemm(const int8_t *W, const float *ws, int N, int K, co
 // mean_cols, the caller's estimate of a group's columns, picks 16 or 32
 // columns per tile; a group's tiles spread over the grid's y, about twice the
 // mean's (blocks past a group's tiles exit at once, the tiles past the grid
-// are walked).  With bank3, two GEMMs over the same columns and groups (an
-// expert's w1 and w3 banks, both N x K) as jobs of one launch.
-static int mf_grouped(const int8_t *bank, const float *bank_s, float *out, const int8_t *bank3, const float *bank3_s,
-                      float *out3, int N, int K, const int8_t *X, const float *Xs, const int *ng, int max_groups,
-                      const int *gexp, const int *goff, const int *gcnt, const int *list, const int *xmap,
-                      int max_cols, int mean_cols, int out_stride, hipStream_t st) {
-    if (N < 1 || K < 32 || (K & 31) || max_groups < 1 || max_cols < 1 || out_stride < N) return -1;
-    const MfCols c{gexp, goff, gcnt, list, xmap, ng};
-    const bool tiled = mft_ok(N, K, max_cols * MAX_TOPK);
-    const int t = mean_cols <= 16 ? MFT_32x16 : MFT_32x32, tr = tiled ? mft_tile_rows(t) : MF_ROWS;
-    const int nrt = (N + tr - 1) / tr;
-    MfJobs jobs{};
-    if (bank3) {
-        jobs.j[0] = MfJob{bank, bank_s, out, X, Xs, N, out_stride, 0, K};
-        jobs.j[1] = MfJob{bank3, bank3_s, out3, X, Xs, N, out_stride, nrt, K};
-        jobs.n = 2;
-    }
-    if (tiled) {
-        const int tc = mft_tile_cols(t), most = (max_cols + tc - 1) / tc, ys = 2 + 2 * mean_cols / tc;
-        mft_launch(t, dim3(bank3 ? 2 * nrt : nrt, ys < most ? ys : most, max_groups), bank, bank_s, N, K, (size_t)N * K,
-                   X, Xs, 0, c, out, out_stride, jobs, st);
-    } else {
-        hipLaunchKernelGGL(k_mfma_q8, dim3(bank3 ? 2 * nrt : nrt, 1, max_groups), dim3(MF_THREADS), 0, st, bank,
-                           bank_s, N, K, (size_t)N * K, X, Xs, 0, c, out, out_stride, jobs);
-    }
-    return (int)hipGetLastError();
+// are walked).
+static int mf_grouped_y(int max_cols, int mean_cols, int tc) {
+    const int most = (max_cols + tc - 1) / tc, ys = 2 + 2 * mean_cols / tc;
+    return ys < most ? ys : most;
 }
 extern "C" int l98k_mfma_gemm_grouped(const int8_t *bank, const float *bank_s, int N, int K, const int8_t *X,
                                       const float *Xs, const int *ng, int max_groups, const int *gexp,
                                       const int *goff, const int *gcnt, const int *list, const int *xmap,
                                       int max_cols, int mean_cols, float *out, int out_stride, hipStream_t st) {
-    return mf_grouped(bank, bank_s, out, nullptr, nullptr, nullptr, N, K, X, Xs, ng, max_groups, gexp, goff, gcnt,
-                      list, xmap, max_cols, mean_cols, out_stride, st);
+    if (N < 1 || K < 32 || (K & 31) || max_groups < 1 || max_cols < 1 || out_stride < N) return -1;
+    const MfCols c{gexp, goff, gcnt, list, xmap, ng};
+    if (mft_ok(N, K, max_cols * MAX_TOPK)) {
+        const int t = mean_cols <= 16 ? MFT_32x16 : MFT_32x32, tr = mft_tile_rows(t), tc = mft_tile_cols(t);
+        mft_launch(t, dim3((N + tr - 1) / tr, mf_grouped_y(max_cols, mean_cols, tc), max_groups), bank, bank_s, N, K,
+                   (size_t)N * K, X, Xs, 0, c, out, out_stride, MfJobs{}, st);
+    } else {
+        hipLaunchKernelGGL(k_mfma_q8, dim3((N + MF_ROWS - 1) / MF_ROWS, 1, max_groups), dim3(MF_THREADS), 0, st, bank,
+                           bank_s, N, K, (size_t)N * K, X, Xs, 0, c, out, out_stride, MfJobs{});
+    }
+    return (int)hipGetLastError();
 }
-extern "C" int l98k_mfma_gemm_grouped2(const int8_t *bank1, const float *bank1_s, float *out1, const int8_t *bank3,
-                                       const float *bank3_s, float *out3, int N, int K, const int8_t *X,
-                                       const float *Xs, const int *ng, int max_groups, const int *gexp,
-                                       const int *goff, const int *gcnt, const int *list, const int *xmap,
-                                       int max_cols, int mean_cols, int out_stride, hipStream_t st) {
-    if (!bank3) return -1;
-    return mf_grouped(bank1, bank1_s, out1, bank3, bank3_s, out3, N, K, X, Xs, ng, max_groups, gexp, goff, gcnt, list,
-                      xmap, max_cols, mean_cols, out_stride, st);
+
+// The experts' first half over `pairs` rows (group columns name them): silu(w1
+// x) * w3 x, both banks N x K, quantized per 32 into q [pairs][N] and qs.  On
+// the tiled kernel one launch (PAIR); else the two GEMMs into h1 and h3
+// (scratch [pairs][N]) and the quantizing producer.  One launch instead of
+// two jobs of one and the producer's: 32 sessions of 4 rows at d = 2048, 24 +
+// 5.3 -> 20.8 us per layer.
+extern "C" int l98k_mfma_gemm_pair(const int8_t *bank1, const float *bank1_s, const int8_t *bank3,
+                                   const float *bank3_s, int N, int K, const int8_t *X, const float *Xs, const int *ng,
+                                   int max_groups, const int *gexp, const int *goff, const int *gcnt, const int *list,
+                                   const int *xmap, int max_cols, int mean_cols, int pairs, float *h1, float *h3,
+                                   int8_t *q, float *qs, hipStream_t st) {
+    if (N < 32 || (N & 31) || K < 32 || (K & 31) || max_groups < 1 || max_cols < 1 || pairs < 1) return -1;
+    if (mft_ok(N, K, max_cols * MAX_TOPK)) {
+        const MfCols c{gexp, goff, gcnt, list, xmap, ng};
+        const MfPair p{bank3, bank3_s, q, qs};
+        const bool narrow = mean_cols <= 16;
+        const dim3 grid(N / 32, mf_grouped_y(max_cols, mean_cols, narrow ? 16 : 32), max_groups);
+        if (narrow)
+            hipLaunchKernelGGL((k_mfma_q8t<2, 1, 2, 1, true>), grid, dim3(128), 0, st, bank1, bank1_s, N, K,
+                               (size_t)N * K, X, Xs, 0, c, nullptr, 0, MfJobs{}, p);
+        else
+            hipLaunchKernelGGL((k_mfma_q8t<2, 1, 2, 2, true>), grid, dim3(256), 0, st, bank1, bank1_s, N, K,
+                               (size_t)N * K, X, Xs, 0, c, nullptr, 0, MfJobs{}, p);
+        return (int)hipGetLastError();
+    }
+    int rc = l98k_mfma_gemm_grouped(bank1, bank1_s, N, K, X, Xs, ng, max_groups, gexp, goff, gcnt, list, xmap, max_cols,
+                                    mean_cols, h1, N, st);
+    if (!rc)
+        rc = l98k_mfma_gemm_grouped(bank3, bank3_s, N, K, X, Xs, ng, max_groups, gexp, goff, gcnt, list, xmap,
+                                    max_cols, mean_cols, h3, N, st);
+    return rc ? rc : l98k_wide_pro(1, h1, h3, N, nullptr, nullptr, 0, N, pairs, q, qs, st);
 }
 
 static bool wide_pro_ok(int mode, int src_stride, const int *sel_idx, const float *sel_w, int topk, int n, int rows) {
