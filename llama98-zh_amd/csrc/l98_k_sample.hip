@@ -166,11 +166,12 @@ __device__ __forceinline__ bool xp_near(float A, float An) {
 // batch issued before the first use.
 #define XP_BATCH 8
 // vec: the row is 16-byte aligned and CH a multiple of 4, so a batch is
-// four 16-byte loads per thread (XP_BATCH * 2 elements)
+// eight 16-byte loads per thread (XP_BATCH * 4 elements: a whole 128-byte
+// line of the thread's own at the usual row lengths)
 template <class G, class F>
 __device__ __forceinline__ void xp_walk(const G &get, int i0, int CH, bool vec, const bool &stop, F f) {
     if (vec) {
-        constexpr int B = 2 * XP_BATCH;
+        constexpr int B = 4 * XP_BATCH;
         for (int k0 = 0; k0 < CH && !stop; k0 += B) {
             float4 v[B / 4];
 #pragma unroll
@@ -342,14 +343,28 @@ __device__ __forceinline__ void xprefix(const G &get, int n, int mode, float c, 
         __syncthreads();
         return;
     }
-    // every element's exact prefix; the first one past c
-    int best = 0x7FFFFFFF;
-    float bestv = 0.0f;
-    {
+    // The prefixes do not decrease, so the first one past c is in the chunk of
+    // the first thread whose last prefix is past c; that thread walks it.
+    // (Every thread walking its own chunk and comparing every prefix: the draw
+    // at n = 65536 58 us, this 50.  A sum that turns NaN took the serial loop.)
+    const uint32_t rk0 = L.cnt_ex[tid];
+    const unsigned long long qp0 = L.q_ex[tid];
+    auto value = [&](uint32_t rk, unsigned long long qp) {
+        const XRec r = L.rec[rk];
+        const int E = (int)(r.info & 255u), eb = E > 1 ? E : 1;
+        const unsigned long long run = qp - (((unsigned long long)r.b << 32) | r.a);
+        return L.sA[rk] + (float)run * __builtin_amdgcn_ldexpf(1.0f, eb - 150);
+    };
+    const float last = value(rk0 + cnt, qp0 + qs);
+    const int first = blk_min_i32((mode == XP_FIRST_GT ? c < last : last >= c) ? tid : 0x7FFFFFFF, L);
+    if (first == 0x7FFFFFFF) {
+        if (tid == 0) { L.result = -1; L.fres = L.sE[K]; }
+    } else if (tid == first) {
         float A = off;
-        int E0 = f_binade(off);
-        uint32_t rk = L.cnt_ex[tid];
-        unsigned long long qp = L.q_ex[tid];
+        int E0 = f_binade(off), best = -1;
+        uint32_t rk = rk0;
+        unsigned long long qp = qp0;
+        float bestv = 0.0f;
         bool found = false;
         xp_walk(get, i0, CH, vec, found, [&](int k, float x) {
             const int i = i0 + k;
@@ -357,28 +372,16 @@ __device__ __forceinline__ void xprefix(const G &get, int n, int mode, float c, 
             const int E1 = f_binade(An);
             uint32_t q;
             const uint32_t plain = ps_classify(x, E0, xp_near(A, An) ? -1 : E1, &q);
-            float pref;
-            if (!plain) {
-                rk++;
-                pref = L.sA[rk];
-            } else {
-                qp += q;
-                const XRec r = L.rec[rk];
-                const int E = (int)(r.info & 255u), eb = E > 1 ? E : 1;
-                const unsigned long long run = qp - (((unsigned long long)r.b << 32) | r.a);
-                pref = L.sA[rk] + (float)run * __builtin_amdgcn_ldexpf(1.0f, eb - 150);
-            }
+            if (!plain) rk++;
+            qp += q;
+            const float pref = plain ? value(rk, qp) : L.sA[rk];
             const bool hit = i < n && (mode == XP_FIRST_GT ? c < pref : pref >= c);
             if (hit) { best = i; bestv = pref; found = true; }
             A = An;
             E0 = E1;
         });
-    }
-    const int first = blk_min_i32(best, L);
-    if (best == first && first != 0x7FFFFFFF) L.fres = bestv;
-    if (tid == 0) {
-        L.result = first == 0x7FFFFFFF ? -1 : first;
-        if (first == 0x7FFFFFFF) L.fres = L.sE[K];
+        L.result = best;
+        L.fres = bestv;
     }
     __syncthreads();
 }
