@@ -18,10 +18,11 @@
 // bytes each, and receives D[4 (l / 16) + v][l % 16] in result register v.
 // A is the weight tile (rows), B the activation tile (tokens).
 //
-// Two kernels: k_mfma_q8t for K a multiple of 128 (every configuration of
-// bench.py), and k_mfma_q8 for any K (the toy models' 32, 64, 96, ...): blocks
-// of 16 weight rows x 64 token columns (a wave per 16 columns), K through
-// double-buffered LDS stages of MF_KC bytes (eight groups).
+// Three kernels: k_mfma_q8t for K a multiple of 128 (every configuration of
+// bench.py); for any other K (the toy models' 32, 64, 96, ..., an expert width
+// of 704 or 1344) k_mfma_q8, blocks of 16 weight rows x 64 token columns (a wave
+// per 16 columns), K through double-buffered LDS stages of MF_KC bytes (eight
+// groups), and its narrow form k_mfma_q8n, 64 weight rows x 16 token columns.
 #include "l98_devmath.h"
 #include "l98_launch.h"
 
@@ -278,6 +279,174 @@ __global__ __launch_bounds__(MF_THREADS) void k_mfma_q8(const int8_t *__restrict
 
 #undef MF_STAGE_LOAD
 #undef MF_STAGE_PUT
+
+// The narrow form of k_mfma_q8: a block computes 64 weight rows x 16 token
+// columns (wave w: rows 16 w .. 16 w + 15 of the same 16 columns), so each block
+// streams four times the weights of k_mfma_q8's 16-row tile and stages only the
+// 16 columns it uses, and the loads run two stages ahead (register sets A and B
+// alternate) - for few columns per weight tile, where a stage's round trip, not
+// the arithmetic, bounds the block (mf_narrow and the grouped launches say
+// where).  Dense (cols.list null: column t is activation and output row t, t < M;
+// jobs as in k_mfma_q8; a 1-D grid mapped onto the XCDs so that the column tiles
+// of a weight tile share an L2) or grouped (block z is group g; a group's column
+// tiles spread over the grid's y, whose extra blocks exit at once).  Same MFMAs
+// and fold per (row, column) as k_mfma_q8, so the same bits.
+#define MFN_ROWS 64
+#define MFN_COLS 16
+#define MFN_STAGE_LOAD(R, st_)                                                                 \
+    do {                                                                                       \
+        const int off_ = imin((st_) * MF_KC + 16 * pc, K - 16);                                \
+        R##w0 = *reinterpret_cast<const int4 *>(wl0 + off_);                                   \
+        R##w1 = *reinterpret_cast<const int4 *>(wl1 + off_);                                   \
+        R##w2 = *reinterpret_cast<const int4 *>(wl2 + off_);                                   \
+        R##w3 = *reinterpret_cast<const int4 *>(wl3 + off_);                                   \
+        R##x0 = *reinterpret_cast<const int4 *>(xl0 + off_);                                   \
+        if (tid < 64) {                                                                        \
+            const int g_ = (st_) * (MF_KC / 32) + 2 * (tid & 3);                               \
+            R##t0 = xsl[imin(g_, nb - 1)];                                                     \
+            R##t1 = xsl[imin(g_ + 1, nb - 1)];                                                 \
+        }                                                                                      \
+    } while (0)
+#define MFN_STAGE_PUT(R, b_)                                                                   \
+    do {                                                                                       \
+        *reinterpret_cast<int4 *>(&s_w[b_][rr][16 * pc]) = R##w0;                              \
+        *reinterpret_cast<int4 *>(&s_w[b_][rr + 16][16 * pc]) = R##w1;                         \
+        *reinterpret_cast<int4 *>(&s_w[b_][rr + 32][16 * pc]) = R##w2;                         \
+        *reinterpret_cast<int4 *>(&s_w[b_][rr + 48][16 * pc]) = R##w3;                         \
+        *reinterpret_cast<int4 *>(&s_x[b_][rr][16 * pc]) = R##x0;                              \
+        if (tid < 64) *reinterpret_cast<float2 *>(&s_xs[b_][tid >> 2][2 * (tid & 3)]) = make_float2(R##t0, R##t1); \
+    } while (0)
+__global__ __launch_bounds__(MF_THREADS) void k_mfma_q8n(const int8_t *__restrict__ W0, const float *__restrict__ ws0,
+                                                          int N0, int K0, size_t w_group_stride,
+                                                          const int8_t *__restrict__ X0, const float *__restrict__ Xs0,
+                                                          int M, MfCols cols, float *__restrict__ out0,
+                                                          int out_stride0, MfJobs jobs) {
+    __shared__ __align__(16) int8_t s_w[2][MFN_ROWS][MF_LDS_ROW];
+    __shared__ __align__(16) int8_t s_x[2][MFN_COLS][MF_LDS_ROW];
+    __shared__ __align__(16) float s_xs[2][MFN_COLS][MF_KC / 32];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int8_t *W = W0;
+    const float *ws = ws0;
+    float *out = out0;
+    const int8_t *X = X0;
+    const float *Xs = Xs0;
+    int N = N0, K = K0, out_stride = out_stride0, bx = blockIdx.x;
+    int cy = blockIdx.y, cys = gridDim.y;
+    if (!cols.list) {
+        // Dense: a 1-D grid of (row tiles rounded up to 8) x column tiles.
+        // Blocks go to the 8 XCDs in turn by linear index, so block L runs on
+        // XCD L % 8; give XCD x the row tiles x, x + 8, ... with all their
+        // column tiles one after another, so the column tiles that share a
+        // weight tile share that XCD's L2 (weights read from HBM once).
+        const int ny = (M + MFN_COLS - 1) / MFN_COLS, xcd = bx & 7, sl = bx >> 3, q = sl / ny;
+        bx = q * 8 + xcd;
+        cy = sl - q * ny;
+        cys = ny;
+        const int nrt = jobs.n ? jobs.j[jobs.n - 1].blk0 + (jobs.j[jobs.n - 1].N + MFN_ROWS - 1) / MFN_ROWS
+                               : (N0 + MFN_ROWS - 1) / MFN_ROWS;
+        if (bx >= nrt) return;
+    }
+    if (jobs.n) {
+        int ji = 0;
+#pragma unroll
+        for (int k = 1; k < MF_MAX_JOBS; k++)
+            if (k < jobs.n && bx >= jobs.j[k].blk0) ji = k;
+        const MfJob jb = jobs.j[ji];
+        W = jb.W;
+        ws = jb.ws;
+        out = jb.out;
+        X = jb.X;
+        Xs = jb.Xs;
+        K = jb.K;
+        N = jb.N;
+        out_stride = jb.out_stride;
+        bx -= jb.blk0;
+    }
+    int ncols = M, cbase = 0;
+    const int8_t *Wg = W;
+    const float *wsg = ws;
+    if (cols.list) {
+        const int g = blockIdx.z;
+        if (g >= *cols.ng) return;
+        ncols = cols.gcnt[g];
+        cbase = cols.goff[g];
+        const int e = cols.gexp[g];
+        Wg = W + (size_t)e * w_group_stride;
+        wsg = ws + (size_t)e * N;
+    }
+    const int n0 = bx * MFN_ROWS, nb = K >> 5;
+    const int pc = tid & 15, rr = tid >> 4;
+    auto wrow = [&](int j) { const int r = n0 + rr + 16 * j; return Wg + (size_t)(r < N ? r : N - 1) * K; };
+    const int8_t *wl0 = wrow(0), *wl1 = wrow(1), *wl2 = wrow(2), *wl3 = wrow(3);
+    const int kq = 8 * (lane >> 4);
+    const int nst = (K + MF_KC - 1) / MF_KC;
+#pragma unroll 1
+    for (int c0 = cy * MFN_COLS; c0 < ncols; c0 += cys * MFN_COLS) {
+        auto xrow = [&](int c) {
+            const int cc = imin(c0 + c, ncols - 1);
+            if (!cols.list) return cc;
+            const int o = cols.list[cbase + cc];
+            return cols.xmap ? cols.xmap[o] : o;
+        };
+        const int8_t *xl0 = X + (size_t)xrow(rr) * K;                  // column rr's piece pc
+        const float *xsl = Xs + (size_t)xrow(tid >> 2) * nb;            // threads < 64: column tid / 4
+        const int cl = c0 + (lane & 15);
+        int4 Aw0, Aw1, Aw2, Aw3, Ax0, Bw0, Bw1, Bw2, Bw3, Bx0;
+        float At0 = 0.0f, At1 = 0.0f, Bt0 = 0.0f, Bt1 = 0.0f;
+        float f[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        const bool one = nb == 1;
+        float s0 = 0.0f;
+        auto compute = [&](int buf, int st) {
+            const float *sc = s_xs[buf][lane & 15];
+            const v4i_t zero = {0, 0, 0, 0};
+            const int ng = nb - st * (MF_KC / 32);
+#pragma unroll
+            for (int gl = 0; gl < MF_KC / 32; gl++) {
+                if (gl >= ng) break;                               // uniform
+                const long b = *reinterpret_cast<const long *>(&s_x[buf][lane & 15][32 * gl + kq]);
+                const long a = *reinterpret_cast<const long *>(&s_w[buf][16 * wave + (lane & 15)][32 * gl + kq]);
+                const v4i_t dd = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b, zero, 0, 0, 0);
+                mf_fold(f, dd, sc[gl], one);
+            }
+            if (one) s0 = sc[0];
+        };
+        // stage st in buffer st % 2; the loads of stages st + 1 and st + 2
+        // in flight while it runs (stages past the last reload the last)
+        MFN_STAGE_LOAD(A, 0);
+        MFN_STAGE_PUT(A, 0);
+        __syncthreads();
+        MFN_STAGE_LOAD(A, imin(1, nst - 1));
+#pragma unroll 1
+        for (int st = 0; st < nst; st += 2) {
+            MFN_STAGE_LOAD(B, imin(st + 2, nst - 1));
+            __builtin_amdgcn_sched_barrier(0);
+            compute(0, st);
+            MFN_STAGE_PUT(A, 1);
+            __syncthreads();
+            if (st + 1 >= nst) break;                          // uniform
+            MFN_STAGE_LOAD(A, imin(st + 3, nst - 1));
+            __builtin_amdgcn_sched_barrier(0);
+            compute(1, st + 1);
+            MFN_STAGE_PUT(B, 0);
+            __syncthreads();
+        }
+        if (cl < ncols) {
+            float *op = out + (size_t)(cols.list ? cols.list[cbase + cl] : cl) * out_stride;
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int n = n0 + 16 * wave + 4 * (lane >> 4) + v;
+                if (n < N) {
+                    float sum = 0.0f;
+                    if (one) sum = epi_one_group((int)f[v], s0, wsg[n]);
+                    else sum += f[v] * wsg[n];
+                    op[n] = sum;
+                }
+            }
+        }
+    }
+}
+#undef MFN_STAGE_LOAD
+#undef MFN_STAGE_PUT
 
 // The tiled form, for many columns per weight row: a block of four waves (2
 // x 2) computes 32 RT weight rows x 32 CT token columns, a wave 16 RT x 16 CT
@@ -686,6 +855,18 @@ static bool mft_ok(int N, int K, int rows) {
     return K % MFT_KC == 0 && (uint64_t)N * K < (1ull << 32) && (uint64_t)rows * K < (1ull << 32);
 }
 
+// Whether a dense launch of K not a multiple of 128 takes k_mfma_q8n: `blocks`
+// 16-row weight tiles of all its jobs, `stages` the MF_KC-byte stages of those
+// tiles.  Measured (us, rows x K at that many columns, k_mfma_q8n / k_mfma_q8):
+//     2048 x 1056 at  4:  7.2 /  6.8      8192 x  352 at   4:  4.9 /  4.9
+//    16384 x   96 at  4:  3.9 /  5.6     65536 x 1056 at   4: 18.8 / 42.1
+//    65536 x 1056 at 32: 27.5 / 44.2     65536 x  352 at  64: 29.4 / 27.9
+//    16384 x 1056 at 64: 15.6 / 15.3    131072 x 1056 at 128:  172 /  179
+static bool mf_narrow(int M, size_t blocks, size_t stages) {
+    if (M <= 32) return stages >= 1024;
+    return M <= 128 && blocks >= 1024 && stages >= 4 * blocks;
+}
+
 // Several dense GEMMs over the same M rows in one launch: job j multiplies
 // W[j] (N[j] x K[j], scales ws[j]) over the rows of X[j] / Xs[j] into out[j]
 // (row stride out_stride[j]).  The blocks of job j follow those of job
@@ -695,15 +876,18 @@ extern "C" int l98k_mfma_gemm_multi(int n_jobs, const int8_t *const *W, const fl
                                     const int8_t *const *X, const float *const *Xs, int M, hipStream_t st) {
     if (n_jobs < 1 || n_jobs > MF_MAX_JOBS || M < 1) return -1;
     bool tiled = true;
-    size_t rows = 0;
+    size_t rows = 0, tiles16 = 0, stages = 0;
     for (int j = 0; j < n_jobs; j++) {
         if (N[j] < 1 || out_stride[j] < N[j] || K[j] < 32 || (K[j] & 31)) return -1;
         tiled = tiled && mft_ok(N[j], K[j], M);
         rows += (size_t)N[j];
+        tiles16 += (size_t)(N[j] + MF_ROWS - 1) / MF_ROWS;
+        stages += (size_t)(N[j] + MF_ROWS - 1) / MF_ROWS * ((K[j] + MF_KC - 1) / MF_KC);
     }
     int t = M <= 16 ? MFT_32x16 : MFT_32x32;
     if (M > 16 && (rows / 64) * ((M + 31) / 32) >= MFT_BIG) t = MFT_64x32;
-    const int tr = tiled ? mft_tile_rows(t) : MF_ROWS;
+    const bool narrow = !tiled && mf_narrow(M, tiles16, stages);
+    const int tr = tiled ? mft_tile_rows(t) : narrow ? MFN_ROWS : MF_ROWS;
     MfJobs jobs{};
     int blocks = 0;
     for (int j = 0; j < n_jobs; j++) {
@@ -715,6 +899,10 @@ extern "C" int l98k_mfma_gemm_multi(int n_jobs, const int8_t *const *W, const fl
         const int tiles = blocks * ((M + mft_tile_cols(t) - 1) / mft_tile_cols(t));
         mft_launch(t, dim3((tiles + 7) & ~7), W[0], ws[0], N[0], K[0], 0, X[0], Xs[0], M, MfCols{}, out[0],
                    out_stride[0], jobs, st);
+    } else if (narrow) {
+        hipLaunchKernelGGL(k_mfma_q8n, dim3(((blocks + 7) & ~7) * ((M + MFN_COLS - 1) / MFN_COLS)), dim3(MF_THREADS),
+                           0, st, W[0], ws[0], N[0], K[0], (size_t)0, X[0], Xs[0], M, MfCols{}, out[0], out_stride[0],
+                           jobs);
     } else {
         hipLaunchKernelGGL(k_mfma_q8, dim3(blocks, (M + MF_COLS - 1) / MF_COLS), dim3(MF_THREADS), 0, st, W[0], ws[0],
                            N[0], K[0], (size_t)0, X[0], Xs[0], M, MfCols{}, out[0], out_stride[0], jobs);
@@ -738,28 +926,53 @@ static int mf_grouped_y(int max_cols, int mean_cols, int tc) {
     const int most = (max_cols + tc - 1) / tc, ys = 2 + 2 * mean_cols / tc;
     return ys < most ? ys : most;
 }
+// A grouped launch of any K: the bank, or `jobs` banks of the same N and K.  Up
+// to 16 columns in a group (mean_cols) on k_mfma_q8n, but for launches of few
+// tiles.  Its y is odd: with 2 or 4 blocks per row tile the ones past a group's
+// columns, which exit at once, leave the same places of the chip empty in every
+// row of tiles.  Measured (us, groups x rows x K at that many columns each:
+// k_mfma_q8n with 3 or 5 / with 2 or 4 blocks / k_mfma_q8):
+//     16 x  128 x   96 at  8:  4.1 /  4.1 /  3.7
+//     64 x  128 x  704 at  2:  6.2 /  6.1 /  6.7
+//     64 x  512 x  704 at  2:  8.8 / 11.7 / 18.0
+//     64 x  512 x  704 at 16: 10.4 / 21.5 / 19.2
+//    128 x 1024 x 1344 at  8: 38.4 / 57.5 / 98.9
+static int mf_grouped(const int8_t *bank, const float *bank_s, int N, int K, const int8_t *X, const float *Xs,
+                      const MfCols &c, int max_groups, int max_cols, int mean_cols, float *out, int out_stride,
+                      MfJobs jobs, hipStream_t st) {
+    const bool narrow = mean_cols <= 16 && (size_t)max_groups * ((N + MF_ROWS - 1) / MF_ROWS) >= 256;
+    const int tr = narrow ? MFN_ROWS : MF_ROWS, nrt = (N + tr - 1) / tr;
+    for (int j = 0; j < jobs.n; j++) jobs.j[j].blk0 = j * nrt;
+    const int gx = nrt * (jobs.n ? jobs.n : 1);
+    if (narrow)
+        hipLaunchKernelGGL(k_mfma_q8n, dim3(gx, mf_grouped_y(max_cols, mean_cols, MFN_COLS) | 1, max_groups),
+                           dim3(MF_THREADS), 0, st, bank, bank_s, N, K, (size_t)N * K, X, Xs, 0, c, out, out_stride,
+                           jobs);
+    else
+        hipLaunchKernelGGL(k_mfma_q8, dim3(gx, 1, max_groups), dim3(MF_THREADS), 0, st, bank, bank_s, N, K,
+                           (size_t)N * K, X, Xs, 0, c, out, out_stride, jobs);
+    return (int)hipGetLastError();
+}
+
 extern "C" int l98k_mfma_gemm_grouped(const int8_t *bank, const float *bank_s, int N, int K, const int8_t *X,
                                       const float *Xs, const int *ng, int max_groups, const int *gexp,
                                       const int *goff, const int *gcnt, const int *list, const int *xmap,
                                       int max_cols, int mean_cols, float *out, int out_stride, hipStream_t st) {
     if (N < 1 || K < 32 || (K & 31) || max_groups < 1 || max_cols < 1 || out_stride < N) return -1;
     const MfCols c{gexp, goff, gcnt, list, xmap, ng};
-    if (mft_ok(N, K, max_cols * MAX_TOPK)) {
-        const int t = mean_cols <= 16 ? MFT_32x16 : MFT_32x32, tr = mft_tile_rows(t), tc = mft_tile_cols(t);
-        mft_launch(t, dim3((N + tr - 1) / tr, mf_grouped_y(max_cols, mean_cols, tc), max_groups), bank, bank_s, N, K,
-                   (size_t)N * K, X, Xs, 0, c, out, out_stride, MfJobs{}, st);
-    } else {
-        hipLaunchKernelGGL(k_mfma_q8, dim3((N + MF_ROWS - 1) / MF_ROWS, 1, max_groups), dim3(MF_THREADS), 0, st, bank,
-                           bank_s, N, K, (size_t)N * K, X, Xs, 0, c, out, out_stride, MfJobs{});
-    }
+    if (!mft_ok(N, K, max_cols * MAX_TOPK))
+        return mf_grouped(bank, bank_s, N, K, X, Xs, c, max_groups, max_cols, mean_cols, out, out_stride, MfJobs{}, st);
+    const int t = mean_cols <= 16 ? MFT_32x16 : MFT_32x32, tr = mft_tile_rows(t), tc = mft_tile_cols(t);
+    mft_launch(t, dim3((N + tr - 1) / tr, mf_grouped_y(max_cols, mean_cols, tc), max_groups), bank, bank_s, N, K,
+               (size_t)N * K, X, Xs, 0, c, out, out_stride, MfJobs{}, st);
     return (int)hipGetLastError();
 }
 
 // The experts' first half over `pairs` rows (group columns name them): silu(w1
 // x) * w3 x, both banks N x K, quantized per 32 into q [pairs][N] and qs.  On
-// the tiled kernel one launch (PAIR); else the two GEMMs into h1 and h3
-// (scratch [pairs][N]) and the quantizing producer.  One launch instead of
-// two jobs of one and the producer's: 32 sessions of 4 rows at d = 2048, 24 +
+// the tiled kernel one launch (PAIR); else the two GEMMs as two jobs of one into
+// h1 and h3 (scratch [pairs][N]) and the quantizing producer.  One launch instead
+// of those two: 32 sessions of 4 rows at d = 2048, 24 +
 // 5.3 -> 20.8 us per layer.
 extern "C" int l98k_mfma_gemm_pair(const int8_t *bank1, const float *bank1_s, const int8_t *bank3,
                                    const float *bank3_s, int N, int K, const int8_t *X, const float *Xs, const int *ng,
@@ -767,8 +980,8 @@ extern "C" int l98k_mfma_gemm_pair(const int8_t *bank1, const float *bank1_s, co
                                    const int *xmap, int max_cols, int mean_cols, int pairs, float *h1, float *h3,
                                    int8_t *q, float *qs, hipStream_t st) {
     if (N < 32 || (N & 31) || K < 32 || (K & 31) || max_groups < 1 || max_cols < 1 || pairs < 1) return -1;
+    const MfCols c{gexp, goff, gcnt, list, xmap, ng};
     if (mft_ok(N, K, max_cols * MAX_TOPK)) {
-        const MfCols c{gexp, goff, gcnt, list, xmap, ng};
         const MfPair p{bank3, bank3_s, q, qs};
         const bool narrow = mean_cols <= 16;
         const dim3 grid(N / 32, mf_grouped_y(max_cols, mean_cols, narrow ? 16 : 32), max_groups);
@@ -780,11 +993,11 @@ extern "C" int l98k_mfma_gemm_pair(const int8_t *bank1, const float *bank1_s, co
                                (size_t)N * K, X, Xs, 0, c, nullptr, 0, MfJobs{}, p);
         return (int)hipGetLastError();
     }
-    int rc = l98k_mfma_gemm_grouped(bank1, bank1_s, N, K, X, Xs, ng, max_groups, gexp, goff, gcnt, list, xmap, max_cols,
-                                    mean_cols, h1, N, st);
-    if (!rc)
-        rc = l98k_mfma_gemm_grouped(bank3, bank3_s, N, K, X, Xs, ng, max_groups, gexp, goff, gcnt, list, xmap,
-                                    max_cols, mean_cols, h3, N, st);
+    MfJobs jobs{};
+    jobs.j[0] = MfJob{bank1, bank1_s, h1, X, Xs, N, N, 0, K};
+    jobs.j[1] = MfJob{bank3, bank3_s, h3, X, Xs, N, N, 0, K};
+    jobs.n = 2;
+    const int rc = mf_grouped(bank1, bank1_s, N, K, X, Xs, c, max_groups, max_cols, mean_cols, h1, N, jobs, st);
     return rc ? rc : l98k_wide_pro(1, h1, h3, N, nullptr, nullptr, 0, N, pairs, q, qs, st);
 }
 
