@@ -3418,8 +3418,12 @@ int greedy_rounds_batched(const LZModel *mm, LZRunState **states, int n_seq, int
         if (hipMalloc((void **)&w->logits, sizeof(float) * (size_t)R * V) != hipSuccess) return 1;
         w->logits_rows = R;
     }
+    // (the draft steps' items have one row, the verify's K1: past four rows a
+    // context's score rows stop fitting the LDS at half the length)
     const size_t att_item = (size_t)MAX_CHUNK * c.n_heads * (size_t)((max_len + 3) & ~3);
-    if (l98k_attn_items_need_att(c.head_dim, max_len, 1) && w->att_items_floats < att_item * n_seq) {
+    const bool need_att = l98k_attn_items_need_att(c.head_dim, max_len, 1) ||
+                          l98k_attn_items_need_att(c.head_dim, max_len, K1);
+    if (need_att && w->att_items_floats < att_item * n_seq) {
         if (w->att_items) (void)hipFree(w->att_items);
         w->att_items = nullptr;
         w->att_items_floats = 0;

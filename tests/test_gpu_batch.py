@@ -159,3 +159,30 @@ def test_batched_rounds_match_per_session_graphs(pkg, server, echo_model, which)
             for st in groups[g]:
                 eng.free_session(st)
             eng.close()
+
+
+def test_batched_rounds_verify_items_wider_than_draft_items(pkg, model_root):
+    """k = 5 on sessions of 4,608 positions: the draft steps' one-row items keep
+    their score rows in LDS, the verify's six-row items do not fit and go through
+    global memory (128-wide heads; eight score rows fit up to about 3,600
+    positions).  Against each session's own round graph."""
+    from test_gpu_shapes import SHAPES, shape_model
+    SHAPES.setdefault("hd128_long", dict(n_heads=2, n_kv_heads=1, head_dim=128, seq_len=4608))
+    print("[case] batched rounds, k = 5, 4,608 positions", flush=True)
+    eng = pkg.Engine(shape_model(pkg, model_root, "hd128_long"))
+    groups = [[], []]
+    try:
+        need = eng.lib.l98k_attn_items_need_att
+        assert (need(128, 4608, 1), need(128, 4608, 6)) == (0, 1)
+        outs = []
+        for mode, group in enumerate(groups):
+            for i, n in enumerate((30, 700, 19)):
+                group.append(eng.add_session(spec_k_max=5))
+                eng.session_start_on(group[-1], pkg.prompt_tokens(500 + i, n, eng.V))
+            outs.append(eng.greedy_rounds_batch(group, 5, 6, mode=mode)[1])
+        for a, b in zip(*outs):
+            assert np.array_equal(a, b), (a, b)
+    finally:
+        for st in groups[0] + groups[1]:
+            eng.free_session(st)
+        eng.close()
