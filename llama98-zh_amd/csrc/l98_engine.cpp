@@ -825,11 +825,12 @@ struct DState {
     // temperature sampling scratch (allocated on first use)
     char *smp_arena = nullptr;
     float *smp_q = nullptr;                 // [L98_SPEC_K_GPU][V] draft distributions of a round
-    float *smp_p = nullptr, *smp_probs = nullptr;         // [L98_SPEC_K_GPU + 1][V], as the keys and indices
+    float *smp_p = nullptr, *smp_probs = nullptr;         // [depth][V], as the keys and indices
     uint32_t *smp_keys = nullptr, *smp_skeys = nullptr;
     int *smp_svals = nullptr;
     void *smp_tmp = nullptr, *smp_top = nullptr;
     unsigned long long *smp_rng = nullptr;
+    int *smp_ncand = nullptr;               // [depth] top-p candidates of each row
     int *smp_out = nullptr;                 // [16] small results
     float *smp_outf = nullptr;              // [16]
 };
@@ -2502,17 +2503,18 @@ namespace {
 // The temperature sampling scratch of a state, carved from one allocation
 // on first use: the round's draft distributions, the verify rows' target
 // distributions, softmax and top-p candidate keys/indices (sorted copies
-// too), the sort's scratch, the generator state and small results.
+// too), the sort's scratch, the generator state and small results.  A round
+// verifies at most depth rows (its k is below the ring's depth).
 bool smp_ensure(DState *d) {
     if (d->smp_arena) return true;
     const size_t V = (size_t)d->m->c.vocab_size;
-    const int rows = L98_SPEC_K_GPU + 1;
+    const int rows = d->depth;
     const size_t tmp = l98k_smp_sort_tmp_bytes((int)V, rows), W = 4 * V * (size_t)rows;
     size_t off = 0;
     auto take = [&](size_t bytes) { size_t a = off; off = (off + bytes + 255) & ~(size_t)255; return a; };
     const size_t oq = take(sizeof(float) * V * L98_SPEC_K_GPU), op = take(W), opr = take(W), ok = take(W),
                  osk = take(W), osv = take(W), ot = take(tmp), otp = take(l98k_smp_topp_tmp_bytes(rows)),
-                 orng = take(8), oo = take(64), oof = take(64);
+                 onc = take(sizeof(int) * rows), orng = take(8), oo = take(64), oof = take(64);
     char *a = nullptr;
     if (hipMalloc(&a, off) != hipSuccess) return false;
     d->smp_arena = a;
@@ -2524,6 +2526,7 @@ bool smp_ensure(DState *d) {
     d->smp_svals = (int *)(a + osv);
     d->smp_tmp = a + ot;
     d->smp_top = a + otp;
+    d->smp_ncand = (int *)(a + onc);
     d->smp_rng = (unsigned long long *)(a + orng);
     d->smp_out = (int *)(a + oo);
     d->smp_outf = (float *)(a + oof);
@@ -2539,13 +2542,14 @@ bool smp_ensure(DState *d) {
 // skip: a device flag (null: never) that turns every launch into a no-op.
 int dev_target_dist(DState *d, const float *logits, int rows, int V, float temp, float topp,
                     const int *skip = nullptr) {
+    if (rows < 1 || rows > d->depth) return 1;
     const float inv = 1.0f / temp;
     if (!topp_active(topp)) return l98k_smp_softmax(logits, V, rows, inv, d->smp_p, 0.0f, nullptr, nullptr, skip, d->st);
     const float cutoff = (V > 1) ? (1.0f - topp) / (float)(V - 1) : 0.0f;
-    if (l98k_smp_softmax(logits, V, rows, inv, d->smp_probs, cutoff, d->smp_keys, d->smp_out + 8, skip, d->st) ||
+    if (l98k_smp_softmax(logits, V, rows, inv, d->smp_probs, cutoff, d->smp_keys, d->smp_ncand, skip, d->st) ||
         l98k_smp_sort_desc(d->smp_keys, d->smp_skeys, d->smp_svals, V, rows, d->smp_tmp, skip, d->st))
         return 1;
-    return l98k_smp_topp_dist(d->smp_probs, V, rows, d->smp_skeys, d->smp_svals, d->smp_out + 8, topp, d->smp_top,
+    return l98k_smp_topp_dist(d->smp_probs, V, rows, d->smp_skeys, d->smp_svals, d->smp_ncand, topp, d->smp_top,
                               d->smp_p, skip, d->st);
 }
 
@@ -2561,9 +2565,9 @@ int dev_sample_ex(DState *d, const float *row, int V, float temp, float topp, lz
             return 1;
     } else {
         const float cutoff = (V > 1) ? (1.0f - topp) / (float)(V - 1) : 0.0f;
-        if (l98k_smp_softmax(row, V, 1, inv, d->smp_probs, cutoff, d->smp_keys, d->smp_out + 8, nullptr, d->st) ||
+        if (l98k_smp_softmax(row, V, 1, inv, d->smp_probs, cutoff, d->smp_keys, d->smp_ncand, nullptr, d->st) ||
             l98k_smp_sort_desc(d->smp_keys, d->smp_skeys, d->smp_svals, V, 1, d->smp_tmp, nullptr, d->st) ||
-            l98k_smp_sample_topp(d->smp_probs, V, d->smp_skeys, d->smp_svals, d->smp_out + 8, topp, d->smp_rng,
+            l98k_smp_sample_topp(d->smp_probs, V, d->smp_skeys, d->smp_svals, d->smp_ncand, topp, d->smp_rng,
                                  d->smp_out, d->st))
             return 1;
     }

@@ -8,6 +8,7 @@
     the host against the reference's recorded temperature generations (the
     device-resident rounds of l98_generate are checked against the same
     fixtures in test_gpu_golden.py)."""
+import ctypes as C
 import json
 import os
 
@@ -70,5 +71,36 @@ def test_host_temperature_rounds_match_fixture(pkg, model_root, fname):
         assert len(bad) == 0, f"first divergence at token {bad[0]}"
         assert list(ke) == g["k_eff"] and list(na) == g["n_accept"]
         assert eng.last_rng == g["rng"]
+    finally:
+        eng.close()
+
+
+@pytest.mark.parametrize("k", [1, 6])
+def test_sampling_scratch_follows_the_state(pkg, model_root, k):
+    """The sampling scratch of a state (taken at its first temperature call) holds
+    the rows its own ring can verify, k + 1, not the widest draft's: per row the
+    target distribution, softmax, keys and indices with their sorted copies, the
+    sort's indices and its tables (V / 1024 tiles of 1024 digits), beside seven
+    draft distributions."""
+    path = os.path.join(model_root, "micro_v131072")
+    if not os.path.exists(os.path.join(path, "model.bin")):
+        cfg = pkg.synth_config(10)
+        cfg.vocab = 131072
+        pkg.write_model(path, 10, 5, cfg=cfg)
+    print(f"[case] sampling scratch, V = 131072, k = {k}", flush=True)
+    eng = pkg.Engine(path, spec_k_max=k)
+    hip, free, total = C.CDLL("libamdhip64.so"), C.c_size_t(), C.c_size_t()
+
+    def left():
+        assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+    try:
+        prompt = pkg.prompt_tokens(1, 12, eng.V)
+        eng.session_start(prompt)                        # a greedy session: everything else is there
+        before = left()
+        eng.generate(prompt, k, 8, temp=0.8, topp=0.95, seed=3)
+        taken = before - left()
+        want = 4 * eng.V * (7 + 7 * (k + 1))
+        assert taken < want + (6 << 20), (taken, want)   # (allocations are rounded up to 2 MB; a captured round's graph)
     finally:
         eng.close()
