@@ -809,8 +809,8 @@ struct DState {
     int amax_cap = 0;
     int *amax_tok = nullptr;
     int amax_mode = 0;
-    DevCtl *ctl_pinned = nullptr;
     char *mirrors = nullptr;                // the LZRunState's host mirrors (mirrors_alloc)
+    DevCtl *ctl_host = nullptr;             // in the same block: ctl's read-back copy
     bool mirrors_pinned = false;
     int cap_rows = 0;                       // rows of hcap / tokbuf
     RoundRec *hist = nullptr;               // device round records
@@ -1027,9 +1027,9 @@ int chain_put(DState *d, const LZRunState *s) {
     return 0;
 }
 int ctl_get(DState *s, DevCtl *h) {
-    CK(hipMemcpyAsync(s->ctl_pinned, s->ctl, sizeof(DevCtl), hipMemcpyDeviceToHost, s->st));
+    CK(hipMemcpyAsync(s->ctl_host, s->ctl, sizeof(DevCtl), hipMemcpyDeviceToHost, s->st));
     CK(hipStreamSynchronize(s->st));
-    *h = *s->ctl_pinned;
+    *h = *s->ctl_host;
     return 0;
 }
 
@@ -1773,35 +1773,32 @@ int mtp_prefill_dev(DState *s, const float *h, const int *toks, int n, const int
 }  // namespace
 
 namespace {
-// The run state's host mirrors, zeroed, in one block of pinned memory: a
-// device copy into pageable memory is staged piece by piece on the calling
-// thread (measured: the 67 MB of logits of a 32-session verify of 4 rows at V
-// = 131072 take 4.9 ms, 1.0 MB of a 4-row verify at V = 65536 0.32 ms alone),
-// into pinned memory it runs at the link's rate (1.3 ms and 0.03 ms).
-// Non-coherent (only copies write it, and the stream is waited for before it
-// is read), and cleared by the device: the host's first touch of 2.9 MB takes
-// 1.1 ms of page faults, which it now takes only for the pages it reads.
-// Pageable when the host has no memory to pin.
+// The run state's host mirrors, zeroed, and the control block's read-back copy,
+// in one block of pinned memory: a device copy into pageable memory is staged
+// piece by piece on the calling thread (measured: the 67 MB of logits of a
+// 32-session verify of 4 rows at V = 131072 take 4.9 ms, 1.0 MB of a 4-row verify
+// at V = 65536 0.32 ms alone), into pinned memory it runs at the link's rate (1.3
+// ms and 0.03 ms).  Non-coherent (only copies write it, and the stream is waited
+// for before it is read), and cleared by the device, at the link's rate (60 us
+// for 2.7 MB) while the host goes on: the caller waits for d->st.  (The host's
+// first touch of 2.7 MB takes 1.0 ms of page faults, which it now takes only for
+// the pages it reads.)  Pageable when the host has no memory to pin.
 bool mirrors_alloc(LZRunState *s, DState *d, const LZModelConfig &c) {
     const size_t V = (size_t)c.vocab_size, H = (size_t)c.hidden_size, rows = L98_SPEC_K_GPU + 1;
     size_t off = 0;
-    auto take = [&](size_t floats) { const size_t o = off; off = (off + 4 * floats + 255) & ~(size_t)255; return o; };
-    const size_t ol = take(V), om = take(rows * V), oh = take(rows * H), oc = take(H), od = take(V),
-                 ok = take(c.mtp_n_draft > 1 ? LZ_SPEC_K_MAX * V : 0);
+    auto take = [&](size_t bytes) { const size_t o = off; off = (off + bytes + 255) & ~(size_t)255; return o; };
+    const size_t octl = take(sizeof(DevCtl)), ol = take(4 * V), om = take(4 * rows * V), oh = take(4 * rows * H),
+                 oc = take(4 * H), od = take(4 * V), ok = take(c.mtp_n_draft > 1 ? 4 * LZ_SPEC_K_MAX * V : 0);
     d->mirrors_pinned = hipHostMalloc((void **)&d->mirrors, off, hipHostMallocPortable | hipHostMallocNonCoherent) ==
                         hipSuccess;
     if (!d->mirrors_pinned) {
         (void)hipGetLastError();
-        d->mirrors = (char *)malloc(off);
+        d->mirrors = (char *)calloc(off, 1);
     }
     if (!d->mirrors) return false;
-    if (d->mirrors_pinned) {
-        if (hipMemsetAsync(d->mirrors, 0, off, d->st) != hipSuccess || hipStreamSynchronize(d->st) != hipSuccess)
-            return false;
-    } else {
-        memset(d->mirrors, 0, off);
-    }
+    if (d->mirrors_pinned && hipMemsetAsync(d->mirrors, 0, off, d->st) != hipSuccess) return false;
     char *b = d->mirrors;
+    d->ctl_host = (DevCtl *)(b + octl);
     s->logits = (float *)(b + ol);
     s->mtp_logits = (float *)(b + om);
     s->mtp_verify_hidden = (float *)(b + oh);
@@ -1842,26 +1839,28 @@ extern "C" int lz_state_alloc(LZRunState *s, const LZModel *mm, int seq_len, int
         return 1;
     }
     carve(d);
-    if (hipStreamCreateWithFlags(&d->st, hipStreamNonBlocking) != hipSuccess ||
-        hipHostMalloc((void **)&d->ctl_pinned, sizeof(DevCtl), hipHostMallocDefault) != hipSuccess ||
-        hipEventCreate(&d->ev0) != hipSuccess || hipEventCreate(&d->ev1) != hipSuccess ||
-        hipEventCreate(&d->ph[0]) != hipSuccess || hipEventCreate(&d->ph[1]) != hipSuccess ||
-        hipEventCreate(&d->ph[2]) != hipSuccess || hipEventCreate(&d->ph[3]) != hipSuccess) {
-        set_err(errbuf, errlen, "HIP stream/event setup failed");
-        (void)hipFree(d->arena);
-        delete d;
+    s->impl = d;                                // (from here lz_state_free gives everything back)
+    if (hipStreamCreateWithFlags(&d->st, hipStreamNonBlocking) != hipSuccess) {
+        set_err(errbuf, errlen, "HIP stream setup failed");
+        lz_state_free(s);
         return 1;
     }
-    s->impl = d;
-    s->seq_len = d->seq_len;
-    s->ssm_ring_depth = d->depth;
-    s->nt_cap = 4;
-    s->bytes_device = (long long)d->arena_size;
     if (!mirrors_alloc(s, d, c)) {
         set_err(errbuf, errlen, "no host memory for the logits mirrors");
         lz_state_free(s);
         return 1;
     }
+    bool ev = hipEventCreate(&d->ev0) == hipSuccess && hipEventCreate(&d->ev1) == hipSuccess;
+    for (hipEvent_t &e : d->ph) ev = ev && hipEventCreate(&e) == hipSuccess;
+    if (!ev) {
+        set_err(errbuf, errlen, "HIP event setup failed");
+        lz_state_free(s);
+        return 1;
+    }
+    s->seq_len = d->seq_len;
+    s->ssm_ring_depth = d->depth;
+    s->nt_cap = 4;
+    s->bytes_device = (long long)d->arena_size;
     lz_state_reset(s, mm);
     return 0;
 }
@@ -1873,7 +1872,6 @@ extern "C" void lz_state_free(LZRunState *s) {
         if (d->st) (void)hipStreamSynchronize(d->st);
         if (d->arena) (void)hipFree(d->arena);
         if (d->smp_arena) (void)hipFree(d->smp_arena);
-        if (d->ctl_pinned) (void)hipHostFree(d->ctl_pinned);
         if (d->ev0) (void)hipEventDestroy(d->ev0);
         if (d->ev1) (void)hipEventDestroy(d->ev1);
         for (hipEvent_t e : d->ph)
