@@ -272,8 +272,10 @@ int l98_greedy_rounds_ex(const LZModel *m, LZRunState *s, int k, int n_rounds, i
                          int cap, int *n_accept_out, int *experts_out, int *new_pos_out, float *device_ms);
 /* Session batches (configs[4]'s server-style verify).  No counterpart in the
  * reference, which keeps one sequence per LZRunState and has no batching;
- * the reference-equivalent result is n_seq independent calls.  Each session
- * is enqueued on its own stream and the calls return when all are done.
+ * the reference-equivalent result is n_seq independent calls.  The many-row
+ * forward runs on the first session's stream; a model it does not carry
+ * (SubLN, grouped scales) has each session enqueued on its own.  The calls
+ * return when all are done.
  *
  * l98_verify_batch: lz_forward_verify (src/forward.h:2060) of n_tok
  * tokens for each of n_seq sessions of one model; session i verifies

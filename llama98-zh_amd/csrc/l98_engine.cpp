@@ -132,8 +132,35 @@ struct DLayer {
     float *fn_gate = nullptr, *fn_up = nullptr, *fn_down = nullptr;
 };
 
+// Pinned blocks of a model's freed sessions, for its next ones (mirrors_alloc):
+// all of one size, at most MIRROR_POOL_BYTES of them.  Held by the model and by
+// every session, so a session may outlive its model; the last one frees the rest.
+#define MIRROR_POOL_BYTES (32u << 20)
+struct MirrorPool {
+    std::mutex mu;
+    std::vector<char *> blocks;
+    char *take() {
+        std::lock_guard<std::mutex> g(mu);
+        if (blocks.empty()) return nullptr;
+        char *p = blocks.back();
+        blocks.pop_back();
+        return p;
+    }
+    void give(char *p, size_t bytes) {
+        {
+            std::lock_guard<std::mutex> g(mu);
+            if ((blocks.size() + 1) * bytes <= MIRROR_POOL_BYTES) { blocks.push_back(p); return; }
+        }
+        (void)hipHostFree(p);
+    }
+    ~MirrorPool() {
+        for (char *p : blocks) (void)hipHostFree(p);
+    }
+};
+
 struct DModel {
     LZModelConfig c{};
+    std::shared_ptr<MirrorPool> mirrors = std::make_shared<MirrorPool>();
     char *arena = nullptr;
     size_t arena_size = 0, arena_used = 0;
     DMat embed;
@@ -811,7 +838,9 @@ struct DState {
     int amax_mode = 0;
     char *mirrors = nullptr;                // the LZRunState's host mirrors (mirrors_alloc)
     DevCtl *ctl_host = nullptr;             // in the same block: ctl's read-back copy
+    size_t mirrors_bytes = 0;
     bool mirrors_pinned = false;
+    std::shared_ptr<MirrorPool> pool;       // the model's
     int cap_rows = 0;                       // rows of hcap / tokbuf
     RoundRec *hist = nullptr;               // device round records
     int hist_cap = 0;
@@ -1782,15 +1811,20 @@ namespace {
 // for before it is read), and cleared by the device, at the link's rate (60 us
 // for 2.7 MB) while the host goes on: the caller waits for d->st.  (The host's
 // first touch of 2.7 MB takes 1.0 ms of page faults, which it now takes only for
-// the pages it reads.)  Pageable when the host has no memory to pin.
+// the pages it reads.)  A block of 2.7 MB takes 0.35 ms to pin and 5.5 MB 0.6, so
+// a freed session's goes to the next (its stream was waited for); pageable when
+// the host has no memory to pin.
 bool mirrors_alloc(LZRunState *s, DState *d, const LZModelConfig &c) {
     const size_t V = (size_t)c.vocab_size, H = (size_t)c.hidden_size, rows = L98_SPEC_K_GPU + 1;
     size_t off = 0;
     auto take = [&](size_t bytes) { const size_t o = off; off = (off + bytes + 255) & ~(size_t)255; return o; };
     const size_t octl = take(sizeof(DevCtl)), ol = take(4 * V), om = take(4 * rows * V), oh = take(4 * rows * H),
                  oc = take(4 * H), od = take(4 * V), ok = take(c.mtp_n_draft > 1 ? 4 * LZ_SPEC_K_MAX * V : 0);
-    d->mirrors_pinned = hipHostMalloc((void **)&d->mirrors, off, hipHostMallocPortable | hipHostMallocNonCoherent) ==
-                        hipSuccess;
+    d->mirrors_bytes = off;
+    d->pool = d->m->mirrors;
+    d->mirrors = d->pool->take();
+    d->mirrors_pinned = d->mirrors || hipHostMalloc((void **)&d->mirrors, off,
+                                                    hipHostMallocPortable | hipHostMallocNonCoherent) == hipSuccess;
     if (!d->mirrors_pinned) {
         (void)hipGetLastError();
         d->mirrors = (char *)calloc(off, 1);
@@ -1808,7 +1842,7 @@ bool mirrors_alloc(LZRunState *s, DState *d, const LZModelConfig &c) {
     return true;
 }
 void mirrors_free(DState *d) {
-    if (d->mirrors_pinned) (void)hipHostFree(d->mirrors);
+    if (d->mirrors_pinned) d->pool->give(d->mirrors, d->mirrors_bytes);
     else free(d->mirrors);
     d->mirrors = nullptr;
 }

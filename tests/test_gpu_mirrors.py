@@ -1,6 +1,9 @@
 """A run state's host mirrors (pinned, written by device copies): every call has
-written what it returns through them by the time it returns."""
+written what it returns through them by the time it returns; and their blocks
+pass from freed sessions to new ones cleared, across threads, and outlive the
+model."""
 import ctypes as C
+import threading
 
 import numpy as np
 import pytest
@@ -63,3 +66,47 @@ def test_calls_write_their_mirrors_before_they_return(pkg, request, which):
                 assert np.isfinite(got[0][f]).all() and same_bits(got[0][f], got[1][f]), (name, f)
     finally:
         eng.close()
+
+
+def test_blocks_of_freed_sessions_come_back_cleared(pkg, micro):
+    eng = pkg.Engine(micro)
+    print("[case] mirrors of new sessions after freed ones", flush=True)
+
+    def dirty_and_check():
+        st = eng.add_session(seq_len=64)
+        for a in mirrors(pkg, eng, st, True).values():
+            assert not a.any()
+            a.fill(7.0)
+        return st
+    try:
+        for _ in range(3):
+            held = [dirty_and_check() for _ in range(5)]
+            for st in held:
+                eng.free_session(st)
+        bad = []
+
+        def churn():
+            try:
+                for _ in range(8):
+                    eng.free_session(dirty_and_check())
+            except Exception as e:       # noqa: BLE001
+                bad.append(e)
+        threads = [threading.Thread(target=churn) for _ in range(4)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert not bad, bad
+    finally:
+        eng.close()
+
+
+def test_a_session_may_be_freed_after_its_model(pkg, micro):
+    eng = pkg.Engine(micro)
+    print("[case] sessions freed after the model", flush=True)
+    held = [eng.add_session(seq_len=64) for _ in range(3)]
+    eng.free_session(held.pop())
+    eng.close()                          # the model goes
+    for st in held:
+        assert not mirror(st, "logits", 16).any()
+        eng.free_session(st)
