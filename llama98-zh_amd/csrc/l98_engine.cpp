@@ -2568,21 +2568,20 @@ bool smp_ensure(DState *d) {
 // lz_target_dist (top-k and min-p off, src/sampler.c:682-730) of `rows`
 // device logits rows into d->smp_p (a verify's rows together: none depends on
 // another's acceptance, and each launch's one block per row leaves the chip
-// to the others): softmax(row / T), then with top-p the
-// candidates >= (1 - top_p) / (V - 1) sorted by probability (stable), the
-// prefix up to the first cumulative mass >= top_p renormalized.
-// skip: a device flag (null: never) that turns every launch into a no-op.
-int dev_target_dist(DState *d, const float *logits, int rows, int V, float temp, float topp,
-                    const int *skip = nullptr) {
+// to the others; rows past the first rejection are computed and not read):
+// softmax(row / T), then with top-p the candidates >= (1 - top_p) / (V - 1)
+// sorted by probability (stable), the prefix up to the first cumulative mass >=
+// top_p renormalized.
+int dev_target_dist(DState *d, const float *logits, int rows, int V, float temp, float topp) {
     if (rows < 1 || rows > d->depth) return 1;
     const float inv = 1.0f / temp;
-    if (!topp_active(topp)) return l98k_smp_softmax(logits, V, rows, inv, d->smp_p, 0.0f, nullptr, nullptr, skip, d->st);
+    if (!topp_active(topp)) return l98k_smp_softmax(logits, V, rows, inv, d->smp_p, 0.0f, nullptr, nullptr, d->st);
     const float cutoff = (V > 1) ? (1.0f - topp) / (float)(V - 1) : 0.0f;
-    if (l98k_smp_softmax(logits, V, rows, inv, d->smp_probs, cutoff, d->smp_keys, d->smp_ncand, skip, d->st) ||
-        l98k_smp_sort_desc(d->smp_keys, d->smp_skeys, d->smp_svals, V, rows, d->smp_tmp, skip, d->st))
+    if (l98k_smp_softmax(logits, V, rows, inv, d->smp_probs, cutoff, d->smp_keys, d->smp_ncand, d->st) ||
+        l98k_smp_sort_desc(d->smp_keys, d->smp_skeys, d->smp_svals, V, rows, d->smp_tmp, d->st))
         return 1;
     return l98k_smp_topp_dist(d->smp_probs, V, rows, d->smp_skeys, d->smp_svals, d->smp_ncand, topp, d->smp_top,
-                              d->smp_p, skip, d->st);
+                              d->smp_p, d->st);
 }
 
 // lz_sample_ex for temperature > 0 (src/sampler.c:794-840) on a device
@@ -2592,13 +2591,13 @@ int dev_sample_ex(DState *d, const float *row, int V, float temp, float topp, lz
     const float inv = 1.0f / temp;
     if (hipMemcpyAsync(d->smp_rng, rng, sizeof(lz_u64), hipMemcpyHostToDevice, d->st)) return 1;
     if (!topp_active(topp)) {
-        if (l98k_smp_softmax(row, V, 1, inv, d->smp_probs, 0.0f, nullptr, nullptr, nullptr, d->st) ||
+        if (l98k_smp_softmax(row, V, 1, inv, d->smp_probs, 0.0f, nullptr, nullptr, d->st) ||
             l98k_smp_draw(d->smp_probs, V, d->smp_rng, d->smp_out, nullptr, nullptr, nullptr, d->st))
             return 1;
     } else {
         const float cutoff = (V > 1) ? (1.0f - topp) / (float)(V - 1) : 0.0f;
-        if (l98k_smp_softmax(row, V, 1, inv, d->smp_probs, cutoff, d->smp_keys, d->smp_ncand, nullptr, d->st) ||
-            l98k_smp_sort_desc(d->smp_keys, d->smp_skeys, d->smp_svals, V, 1, d->smp_tmp, nullptr, d->st) ||
+        if (l98k_smp_softmax(row, V, 1, inv, d->smp_probs, cutoff, d->smp_keys, d->smp_ncand, d->st) ||
+            l98k_smp_sort_desc(d->smp_keys, d->smp_skeys, d->smp_svals, V, 1, d->smp_tmp, d->st) ||
             l98k_smp_sample_topp(d->smp_probs, V, d->smp_skeys, d->smp_svals, d->smp_ncand, topp, d->smp_rng,
                                  d->smp_out, d->st))
             return 1;
@@ -2615,7 +2614,7 @@ int dev_sample_ex(DState *d, const float *row, int V, float temp, float topp, lz
 // (lz_sample_temp_q, src/sampler.c:736-747); the (k+1)-row verify; every
 // row's target distribution (lz_target_dist); per row i the acceptance test
 // with residual resampling, which on a rejection records n_accept = i and
-// sets ctl->smp_done, after which every sampling launch of the round does
+// sets ctl->smp_done, after which every draw and acceptance of the round does
 // nothing (the reference's loop stops there, drawing nothing more); the
 // bonus draw from row k when no row rejected; then the ring rollback, chain
 // reseed, catch-up and round record of the greedy round.  Every scalar
@@ -2628,7 +2627,7 @@ int enqueue_temp_round(DState *d, int k, int max_pos, float temp, float topp) {
     for (int i = 0; i < k; i++) {
         float *qi = d->smp_q + (size_t)i * V;
         CK(draft_step(d, d->ctl->tok + i, &d->ctl->mtp_pos, i, max_pos, d->draft_logits, nullptr));
-        CK(l98k_smp_softmax(d->draft_logits, V, 1, inv, qi, 0.0f, nullptr, nullptr, nullptr, d->st));
+        CK(l98k_smp_softmax(d->draft_logits, V, 1, inv, qi, 0.0f, nullptr, nullptr, d->st));
         CK(l98k_smp_draw(qi, V, d->smp_rng, d->smp_out, d->smp_outf, d->ctl->tok + 1 + i, nullptr, d->st));
     }
     CK(forward_chunk(d, d->ctl->tok, k + 1, &d->ctl->anchor_pos, 1, max_pos, d->vhidden, true, d->mtp_logits,
@@ -2785,7 +2784,7 @@ int spec_round_temp(const LZModel *mm, LZRunState *s, int anchor, int anchor_pos
         float *qi = d->smp_q + (size_t)i * V;
         int idx = 0;
         float qidx = 0.0f;
-        if (l98k_smp_softmax(row, V, 1, inv, qi, 0.0f, nullptr, nullptr, nullptr, d->st) ||
+        if (l98k_smp_softmax(row, V, 1, inv, qi, 0.0f, nullptr, nullptr, d->st) ||
             l98k_smp_draw(qi, V, d->smp_rng, d->smp_out, d->smp_outf, d->ctl->tok + 1 + i, nullptr, d->st) ||
             hipMemcpyAsync(&idx, d->smp_out, sizeof(int), hipMemcpyDeviceToHost, d->st) ||
             hipMemcpyAsync(&qidx, d->smp_outf, sizeof(float), hipMemcpyDeviceToHost, d->st) ||
@@ -3003,7 +3002,7 @@ extern "C" int l98_sort_desc(const uint32_t *keys, int n, uint32_t *keys_out, in
     if (!dk.get(keys, sizeof(uint32_t) * (size_t)n) || !dko.get(nullptr, sizeof(uint32_t) * (size_t)n) ||
         !dio.get(nullptr, sizeof(int) * (size_t)n) || !dt.get(nullptr, l98k_smp_sort_tmp_bytes(n, 1)))
         return 1;
-    if (l98k_smp_sort_desc((uint32_t *)dk.p, (uint32_t *)dko.p, (int *)dio.p, n, 1, dt.p, nullptr, nullptr)) return 1;
+    if (l98k_smp_sort_desc((uint32_t *)dk.p, (uint32_t *)dko.p, (int *)dio.p, n, 1, dt.p, nullptr)) return 1;
     return dko.put(keys_out, sizeof(uint32_t) * (size_t)n) && dio.put(idx_out, sizeof(int) * (size_t)n) ? 0 : 1;
 }
 

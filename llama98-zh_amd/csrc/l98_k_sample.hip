@@ -19,10 +19,10 @@
 // this file's own (three passes of 10-bit digits: a candidate key, the bits
 // of a probability in [0, 1], is below 2^30).
 //
-// The kernels a device-resident temperature round runs take `skip`, a
-// device flag (the round's "decided" word): when it is set the launch does
-// nothing, so the acceptance rows after the first rejection consume no
-// random numbers, as the reference's loop stops there.
+// A device-resident temperature round's draws and acceptances take a device
+// flag (the round's "decided" word): when it is set the launch does nothing,
+// so the acceptance rows after the first rejection consume no random numbers,
+// as the reference's loop stops there.
 #include <cstring>
 
 #include "l98_devmath.h"
@@ -470,10 +470,9 @@ __device__ __forceinline__ int blk_argmax(const float *x, int n, SmpLds &L) {
 __global__ __launch_bounds__(SMP_THREADS) void k_smp_softmax(const float *__restrict__ logits, int n, float inv_t,
                                                              float *__restrict__ probs, float cutoff,
                                                              uint32_t *__restrict__ keys,
-                                                             int *__restrict__ n_cand, const int *__restrict__ skip) {
+                                                             int *__restrict__ n_cand) {
     __shared__ SmpLds L;
     __shared__ float tab[32];
-    if (skip && *skip) return;
     logits += (size_t)blockIdx.x * n;
     probs += (size_t)blockIdx.x * n;
     if (keys) keys += (size_t)blockIdx.x * n;
@@ -550,9 +549,8 @@ struct TopP {
 __global__ __launch_bounds__(SMP_THREADS) void k_smp_topp_find(const float *__restrict__ probs, int n,
                                                                const uint32_t *__restrict__ skeys,
                                                                const int *__restrict__ n_cand, float topp,
-                                                               TopP *__restrict__ out, const int *__restrict__ skip) {
+                                                               TopP *__restrict__ out) {
     __shared__ SmpLds L;
-    if (skip && *skip) return;
     const int tid = threadIdx.x, row = blockIdx.x, nc = n_cand[row];
     if (nc <= 0) {
         const int a = blk_argmax(probs + (size_t)row * n, n, L);
@@ -565,9 +563,7 @@ __global__ __launch_bounds__(SMP_THREADS) void k_smp_topp_find(const float *__re
 #define TOPP_TILE 1024
 __global__ __launch_bounds__(TOPP_TILE) void k_smp_topp_fill(int n, const uint32_t *__restrict__ skeys,
                                                              const int *__restrict__ svals,
-                                                             const TopP *__restrict__ top, float *__restrict__ p_out,
-                                                             const int *__restrict__ skip) {
-    if (skip && *skip) return;
+                                                             const TopP *__restrict__ top, float *__restrict__ p_out) {
     const int j = blockIdx.x * TOPP_TILE + threadIdx.x;
     if (j >= n) return;
     const TopP t = top[blockIdx.y];
@@ -680,7 +676,11 @@ __global__ __launch_bounds__(SMP_THREADS) void k_smp_xprefix(const float *__rest
 // element at its digit's start + the tiles before + the count of equal digits
 // before it in its tile (lanes of the same digit found with 10 ballots, then
 // the waves before it).  A launch of one block scanning the table between the
-// two took 25 us per pass.  Digits are taken as 1023 - digit, so the order is
+// two took 25 us per pass.  (Every block reading the whole table is quadratic
+// in n, and still cheaper than that scan up to the largest n: a sort of one row
+// of 65,536 keys 38 us against 105, 262,144 86 against 320, 1,048,576 0.78 ms
+// against 1.24; eight rows of 131,072 158 us against 1,422 one by one.)  Digits
+// are taken as 1023 - digit, so the order is
 // descending; every pass keeps the order of equal digits, so equal keys keep
 // index order.
 #define RS_TILE 1024
@@ -693,10 +693,8 @@ __device__ __forceinline__ int rs_digit(uint32_t key, int shift) {
 }
 
 __global__ __launch_bounds__(RS_TILE) void k_rs_count(const uint32_t *__restrict__ keys, int n, int shift,
-                                                      int *__restrict__ hist, int ntiles,
-                                                      const int *__restrict__ skip) {
+                                                      int *__restrict__ hist, int ntiles) {
     __shared__ int cnt[RS_DIG];
-    if (skip && *skip) return;
     const int tid = threadIdx.x, i = blockIdx.x * RS_TILE + tid;
     cnt[tid] = 0;
     __syncthreads();
@@ -707,11 +705,9 @@ __global__ __launch_bounds__(RS_TILE) void k_rs_count(const uint32_t *__restrict
 
 __global__ __launch_bounds__(RS_TILE) void k_rs_scatter(const uint32_t *__restrict__ keys, const int *__restrict__ vals,
                                                         uint32_t *__restrict__ keys_out, int *__restrict__ vals_out,
-                                                        int n, int shift, const int *__restrict__ hist, int ntiles,
-                                                        const int *__restrict__ skip) {
+                                                        int n, int shift, const int *__restrict__ hist, int ntiles) {
     __shared__ unsigned short wcnt[RS_TILE / 64][RS_DIG];   // per wave: elements of each digit
     __shared__ int base[RS_DIG], wsum[RS_TILE / 64];
-    if (skip && *skip) return;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, i = blockIdx.x * RS_TILE + tid;
     const bool valid = i < n;
     const size_t row = (size_t)blockIdx.y * n;
@@ -781,10 +777,10 @@ extern "C" int l98k_upload_exp_table_smp(const float *tab) {
 }
 
 extern "C" int l98k_smp_softmax(const float *logits, int n, int rows, float inv_t, float *probs, float cutoff,
-                                uint32_t *keys, int *n_cand, const int *skip, hipStream_t st) {
+                                uint32_t *keys, int *n_cand, hipStream_t st) {
     if (n < 1 || rows < 1) return -1;
-    hipLaunchKernelGGL(k_smp_softmax, dim3(rows), dim3(SMP_THREADS), 0, st, logits, n, inv_t, probs, cutoff, keys, n_cand,
-                       skip);
+    hipLaunchKernelGGL(k_smp_softmax, dim3(rows), dim3(SMP_THREADS), 0, st, logits, n, inv_t, probs, cutoff, keys,
+                       n_cand);
     return (int)hipGetLastError();
 }
 
@@ -804,7 +800,7 @@ extern "C" size_t l98k_smp_sort_tmp_bytes(int n, int rows) {
 // their indices 0..n-1: keys_out, vals_out.  keys is overwritten (a pass's
 // buffer); tmp holds l98k_smp_sort_tmp_bytes(n, rows) bytes.
 extern "C" int l98k_smp_sort_desc(uint32_t *keys, uint32_t *keys_out, int *vals_out, int n, int rows, void *tmp,
-                                  const int *skip, hipStream_t st) {
+                                  hipStream_t st) {
     if (n < 1 || n > RS_DIG * RS_TILE || rows < 1 || !tmp) return -1;
     const int ntiles = (n + RS_TILE - 1) / RS_TILE;
     int *hist = reinterpret_cast<int *>(tmp);
@@ -818,10 +814,9 @@ extern "C" int l98k_smp_sort_desc(uint32_t *keys, uint32_t *keys_out, int *vals_
     int *vout[RS_PASSES] = {vals_out, vtmp, vals_out};
     for (int pass = 0; pass < RS_PASSES; pass++) {
         const int shift = pass * RS_BITS;
-        hipLaunchKernelGGL(k_rs_count, dim3(ntiles, rows), dim3(RS_TILE), 0, st, kin[pass], n, shift, hist, ntiles,
-                           skip);
+        hipLaunchKernelGGL(k_rs_count, dim3(ntiles, rows), dim3(RS_TILE), 0, st, kin[pass], n, shift, hist, ntiles);
         hipLaunchKernelGGL(k_rs_scatter, dim3(ntiles, rows), dim3(RS_TILE), 0, st, kin[pass], vin[pass], kout[pass],
-                           vout[pass], n, shift, hist, ntiles, skip);
+                           vout[pass], n, shift, hist, ntiles);
     }
     return (int)hipGetLastError();
 }
@@ -829,13 +824,12 @@ extern "C" int l98k_smp_sort_desc(uint32_t *keys, uint32_t *keys_out, int *vals_
 extern "C" size_t l98k_smp_topp_tmp_bytes(int rows) { return sizeof(TopP) * (size_t)rows; }
 
 extern "C" int l98k_smp_topp_dist(const float *probs, int n, int rows, const uint32_t *skeys, const int *svals,
-                                  const int *n_cand, float topp, void *tmp, float *p_out, const int *skip,
-                                  hipStream_t st) {
+                                  const int *n_cand, float topp, void *tmp, float *p_out, hipStream_t st) {
     if (n < 1 || rows < 1 || !tmp) return -1;
     TopP *t = reinterpret_cast<TopP *>(tmp);
-    hipLaunchKernelGGL(k_smp_topp_find, dim3(rows), dim3(SMP_THREADS), 0, st, probs, n, skeys, n_cand, topp, t, skip);
+    hipLaunchKernelGGL(k_smp_topp_find, dim3(rows), dim3(SMP_THREADS), 0, st, probs, n, skeys, n_cand, topp, t);
     hipLaunchKernelGGL(k_smp_topp_fill, dim3((n + TOPP_TILE - 1) / TOPP_TILE, rows), dim3(TOPP_TILE), 0, st, n, skeys,
-                       svals, t, p_out, skip);
+                       svals, t, p_out);
     return (int)hipGetLastError();
 }
 

@@ -49,16 +49,15 @@ int l98k_wide_pro(int mode, const float *src, const float *src2, int src_stride,
 // quantization (the SubLN routed-up and shared-down inputs).
 int l98k_wide_pro_f(int mode, const float *src, const float *src2, int src_stride, const int *sel_idx,
                     const float *sel_w, int topk, int n, int rows, float *fout, hipStream_t st);
-// Temperature sampling (one block per call; l98_k_sample.hip).
-// The softmax, the sort and the top-p distributions take `rows` rows of n (a
-// row's results at row strides of n, n_cand[row]).
-// The launches that take `skip` (a device flag) do nothing when it is set
-// (null: never).
+// Temperature sampling (l98_k_sample.hip).  The softmax, the sort and the
+// top-p distributions take `rows` rows of n (a row's results at row strides of
+// n, n_cand[row]); the draws and acceptances are one block each.
 // probs = softmax(logits * inv_t); with keys: the top-p candidate keys for
 // l98k_smp_sort_desc and their count.
 int l98k_smp_softmax(const float *logits, int n, int rows, float inv_t, float *probs, float cutoff, uint32_t *keys,
-                     int *n_cand, const int *skip, hipStream_t st);
-// A draw from p by the cdf (rng advanced on the device); ctl_tok optional.
+                     int *n_cand, hipStream_t st);
+// A draw from p by the cdf (rng advanced on the device); ctl_tok optional;
+// skip: a device flag that turns the launch into a no-op when set (null: never).
 int l98k_smp_draw(const float *p, int n, unsigned long long *rng, int *out_tok, float *out_p, int *ctl_tok,
                   const int *skip, hipStream_t st);
 // Scratch bytes of l98k_smp_sort_desc for rows of n keys.
@@ -67,12 +66,12 @@ size_t l98k_smp_sort_tmp_bytes(int n, int rows);
 // radix sort of this library's own, three passes of two launches; keys is
 // overwritten.
 int l98k_smp_sort_desc(uint32_t *keys, uint32_t *keys_out, int *vals_out, int n, int rows, void *tmp,
-                       const int *skip, hipStream_t st);
+                       hipStream_t st);
 // Top-p target distributions from the softmax and the sorted candidates (tmp:
 // l98k_smp_topp_tmp_bytes(rows)).
 size_t l98k_smp_topp_tmp_bytes(int rows);
 int l98k_smp_topp_dist(const float *probs, int n, int rows, const uint32_t *skeys, const int *svals,
-                       const int *n_cand, float topp, void *tmp, float *p_out, const int *skip, hipStream_t st);
+                       const int *n_cand, float topp, void *tmp, float *p_out, hipStream_t st);
 // Speculative acceptance of draft x with residual resampling (u given, or
 // drawn when u is null): out[0] token, out[1] accepted.
 int l98k_smp_accept(const float *p, const float *q, int n, int x, const float *u, unsigned long long *rng, int *out,
