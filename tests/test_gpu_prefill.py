@@ -2,9 +2,11 @@
 grouped expert GEMMs, the KDA rows of a chunk in one launch) at long
 contexts.
 
-* A small model with configs[3]'s attention head size (128) and a 4608
-  context: a 4200-token prompt's captured hidden rows, then a capture and
-  a verify at position 4200, against the CPU restatement, bit for bit.
+* Small models with head sizes 128 (configs[3]'s) and 64 and contexts past
+  the length where eight score rows leave the attention block's LDS, so that
+  a chunk is cut into four-row items: a long prompt's captured hidden rows,
+  then a capture and a verify after it, against the CPU restatement, bit for
+  bit.
 * configs[3] itself (d = 2048, 32 layers, 128 experts top-8): its
   4096-token prompt in 512-row chunks against the same prompt through the
   8-row chunked path (15-token calls), hidden rows and the next verify's
@@ -23,12 +25,17 @@ from test_gpu_shapes import SHAPES, shape_model
 pytestmark = pytest.mark.gpu
 
 SHAPES.setdefault("hd128_long", dict(n_heads=2, n_kv_heads=1, head_dim=128, seq_len=4608))
+SHAPES.setdefault("hd64_long", dict(n_heads=2, n_kv_heads=1, head_dim=64, seq_len=4864))
 
 
-def test_long_prefill_matches_oracle(pkg, model_root):
-    print("[case] prefill 4200 tokens, hd 128 model", flush=True)
-    model = shape_model(pkg, model_root, "hd128_long")
-    n = 4200
+@pytest.mark.parametrize("shape,n", [("hd128_long", 4200), ("hd64_long", 4631)])
+def test_long_prefill_matches_oracle(pkg, model_root, shape, n):
+    """The last chunk in four-row items, ending in one of fewer."""
+    print(f"[case] prefill {n} tokens, {shape} model", flush=True)
+    model = shape_model(pkg, model_root, shape)
+    rows = pkg.hip_lib().l98k_attn_item_rows
+    hd = SHAPES[shape]["head_dim"]
+    assert (rows(hd, 512), rows(hd, n - 1)) == (8, 4) and (n - 1) % 512 > 8 and (n - 1) % 512 % 4
     prompt = pkg.prompt_tokens(5, n, 512)
     eng, ora = pkg.Engine(model), Oracle(model)
     try:
@@ -81,13 +88,12 @@ def test_configs3_prompt_chunking_invariant(pkg, model_root):
 
 
 @pytest.mark.parametrize("n", [63, 64, 65, 97, 130, 600])
-def test_split_prefill_matches_chunked(pkg, server, n):
-    """A wide prefill chunk of 64 or more rows runs in three parts, each on
-    its own stream (part p's layers wait for part p - 1's KDA recurrence and
-    attention), when every part exceeds 8 rows; rows and the next verify's
-    logits equal the 8-row chunked path bit for bit, at part sizes around the
-    split's threshold and rounding, and over two wide chunks (600 rows)."""
-    print(f"[case] split prefill n={n}", flush=True)
+def test_wide_prefill_matches_chunked(pkg, server, n):
+    """A wide prefill chunk's rows and the next verify's logits equal the 8-row
+    chunked path bit for bit, at lengths around whole attention items,
+    recurrence stages and GEMM column tiles (64), and over two wide chunks
+    (600 rows)."""
+    print(f"[case] wide prefill n={n}", flush=True)
     prompt = pkg.prompt_tokens(9, n, 8192)
     eng = pkg.Engine(server)
     other = eng.add_session()

@@ -15,6 +15,8 @@ import os
 import numpy as np
 import pytest
 
+from oracle_lib import Oracle
+
 pytestmark = pytest.mark.gpu
 
 GOLDEN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden")
@@ -104,3 +106,26 @@ def test_sampling_scratch_follows_the_state(pkg, model_root, k):
         assert taken < want + (6 << 20), (taken, want)   # (allocations are rounded up to 2 MB; a captured round's graph)
     finally:
         eng.close()
+
+
+@pytest.mark.parametrize("topp", [0.95, 1.0])
+def test_odd_vocabulary_rounds_match_oracle(pkg, model_root, topp):
+    """Rows of 1,031 logits: past the first, a verify row's distribution, keys and
+    sorted places start off the 16-byte loads' alignment."""
+    path = os.path.join(model_root, "micro_v1031")
+    if not os.path.exists(os.path.join(path, "model.bin")):
+        cfg = pkg.synth_config(10)
+        cfg.vocab = 1031
+        pkg.write_model(path, 10, 6, cfg=cfg)
+    prompt = pkg.prompt_tokens(2, 20, 1031)
+    eng, ora = pkg.Engine(path), Oracle(path)
+    try:
+        for k in (1, 4):
+            print(f"[case] temperature rounds, V = 1031, k = {k}, top-p {topp}", flush=True)
+            got = eng.generate(prompt, k, 24, temp=0.9, topp=topp, seed=11)[0]
+            want = ora.generate(prompt, k, 24, temp=0.9, topp=topp, seed=11)[0]
+            m = min(len(got), len(want))
+            assert m >= 24 and np.array_equal(np.asarray(got[:m]), np.asarray(want[:m])), (got, want)
+    finally:
+        eng.close()
+        ora.close()
