@@ -29,8 +29,7 @@
 typedef int v4i_t __attribute__((ext_vector_type(4)));
 
 #define MF_THREADS 256
-#define MF_RT 1           // 16-row MFMA tiles per wave
-#define MF_ROWS (16 * MF_RT)  // weight rows per block
+#define MF_ROWS 16        // weight rows per block
 #define MF_COLS 64        // token columns per block (16 per wave)
 #define MF_KC 256         // K bytes (eight groups) per LDS stage
 #define MF_LDS_ROW (MF_KC + 16)   // padded stage row: the lanes' 8-byte operand reads spread over the banks
@@ -61,24 +60,16 @@ struct MfCols {
     const int *ng;           // groups actually present (device)
 };
 
-__device__ __forceinline__ long ld8(const int8_t *p) { return *reinterpret_cast<const long *>(p); }
-
-// One LDS stage of k_mfma_q8 in a thread's registers (set R: Aw0 .. At1):
-// its four 16-byte pieces of weight rows and of activation
-// columns, and two of the block's 64 x 8 activation group scales (column
-// tid / 4, groups 2 (tid % 4) and the next).  Plain locals (a struct would
-// be kept in scratch memory across the scheduling barriers that hold the
-// loads' issue in place).
+// One LDS stage of k_mfma_q8 in a thread's registers (set R: Aw0 .. At1): its
+// 16-byte piece of a weight row and four of activation columns, and two of the
+// block's 64 x 8 activation group scales (column tid / 4, groups 2 (tid % 4) and
+// the next).  Plain locals (a struct would be kept in scratch memory across the
+// scheduling barriers that hold the loads' issue in place).
 static_assert(MF_KC == 256 && MF_THREADS == 256, "a stage: eight group scales per column, two per thread");
 #define MF_STAGE_LOAD(R, st_)                                                                  \
     do {                                                                                       \
         const int off_ = imin((st_) * MF_KC + 16 * pc, K - 16);                                \
         R##w0 = *reinterpret_cast<const int4 *>(wl0 + off_);                                   \
-        if constexpr (MF_RT >= 2) R##w1 = *reinterpret_cast<const int4 *>(wl1 + off_);         \
-        if constexpr (MF_RT == 4) {                                                            \
-            R##w2 = *reinterpret_cast<const int4 *>(wl2 + off_);                               \
-            R##w3 = *reinterpret_cast<const int4 *>(wl3 + off_);                               \
-        }                                                                                      \
         R##x0 = *reinterpret_cast<const int4 *>(xl0 + off_);                                   \
         R##x1 = *reinterpret_cast<const int4 *>(xl1 + off_);                                   \
         R##x2 = *reinterpret_cast<const int4 *>(xl2 + off_);                                   \
@@ -90,11 +81,6 @@ static_assert(MF_KC == 256 && MF_THREADS == 256, "a stage: eight group scales pe
 #define MF_STAGE_PUT(R, b_)                                                                    \
     do {                                                                                       \
         *reinterpret_cast<int4 *>(&s_w[b_][rr][16 * pc]) = R##w0;                              \
-        if constexpr (MF_RT >= 2) *reinterpret_cast<int4 *>(&s_w[b_][rr + 16][16 * pc]) = R##w1; \
-        if constexpr (MF_RT == 4) {                                                            \
-            *reinterpret_cast<int4 *>(&s_w[b_][rr + 32][16 * pc]) = R##w2;                     \
-            *reinterpret_cast<int4 *>(&s_w[b_][rr + 48][16 * pc]) = R##w3;                     \
-        }                                                                                      \
         *reinterpret_cast<int4 *>(&s_x[b_][rr][16 * pc]) = R##x0;                              \
         *reinterpret_cast<int4 *>(&s_x[b_][rr + 16][16 * pc]) = R##x1;                         \
         *reinterpret_cast<int4 *>(&s_x[b_][rr + 32][16 * pc]) = R##x2;                         \
@@ -108,36 +94,15 @@ __device__ __forceinline__ void mf_fold(float (&f)[4], v4i_t d, float s, bool on
     f[2] += one ? (float)d[2] : (float)d[2] * s;
     f[3] += one ? (float)d[3] : (float)d[3] * s;
 }
-__device__ __forceinline__ void mf_stage(float (&f)[MF_RT][4], const int8_t (*sw)[MF_LDS_ROW],
-                                         const int8_t (*sx)[MF_LDS_ROW], const float *sc, int ng, bool one,
-                                         int wave, int lane, int kq) {
+__device__ __forceinline__ void mf_stage(float (&f)[4], const int8_t (*sw)[MF_LDS_ROW], const int8_t (*sx)[MF_LDS_ROW],
+                                         const float *sc, int ng, bool one, int wave, int lane, int kq) {
     const v4i_t zero = {0, 0, 0, 0};
 #pragma unroll
     for (int gl = 0; gl < MF_KC / 32; gl++) {
         if (gl >= ng) break;                           // uniform
         const long b = *reinterpret_cast<const long *>(&sx[16 * wave + (lane & 15)][32 * gl + kq]);
-        const long a0 = *reinterpret_cast<const long *>(&sw[(lane & 15)][32 * gl + kq]);
-        const v4i_t d0 = __builtin_amdgcn_mfma_i32_16x16x32_i8(a0, b, zero, 0, 0, 0);
-        const float s = sc[gl];
-        if constexpr (MF_RT == 1) {
-            mf_fold(f[0], d0, s, one);
-            continue;
-        }
-        const long a1 = *reinterpret_cast<const long *>(&sw[16 + (lane & 15)][32 * gl + kq]);
-        const v4i_t d1 = __builtin_amdgcn_mfma_i32_16x16x32_i8(a1, b, zero, 0, 0, 0);
-        if constexpr (MF_RT == 4) {
-            const long a2 = *reinterpret_cast<const long *>(&sw[32 + (lane & 15)][32 * gl + kq]);
-            const long a3 = *reinterpret_cast<const long *>(&sw[48 + (lane & 15)][32 * gl + kq]);
-            const v4i_t d2 = __builtin_amdgcn_mfma_i32_16x16x32_i8(a2, b, zero, 0, 0, 0);
-            const v4i_t d3 = __builtin_amdgcn_mfma_i32_16x16x32_i8(a3, b, zero, 0, 0, 0);
-            mf_fold(f[0], d0, s, one);
-            mf_fold(f[1], d1, s, one);
-            mf_fold(f[MF_RT - 2], d2, s, one);
-            mf_fold(f[MF_RT - 1], d3, s, one);
-        } else {
-            mf_fold(f[0], d0, s, one);
-            mf_fold(f[MF_RT - 1], d1, s, one);
-        }
+        const long a = *reinterpret_cast<const long *>(&sw[(lane & 15)][32 * gl + kq]);
+        mf_fold(f, __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b, zero, 0, 0, 0), sc[gl], one);
     }
 }
 
@@ -196,14 +161,12 @@ __global__ __launch_bounds__(MF_THREADS) void k_mfma_q8(const int8_t *__restrict
         const int cc = cl < ncols ? cl : ncols - 1;
         const int orow = cols.list ? cols.list[cbase + cc] : cc;
         const int kq = 8 * (lane >> 4);
-        // Stage loads: thread t takes the 16-byte piece pc of weight rows
-        // rr + 16 j (j < MF_RT) and activation columns rr + 16 j (j < 4) of
-        // the block: every row's
-        // MF_KC-byte stage is read by 16 consecutive threads.  Rows past N and
-        // columns past ncols repeat the last; pieces past K repeat the row's
-        // last piece (their groups are not used).
+        // Stage loads: thread t takes the 16-byte piece pc of weight row rr and
+        // activation columns rr + 16 j (j < 4) of the block: every row's MF_KC-byte
+        // stage is read by 16 consecutive threads.  Rows past N and columns past
+        // ncols repeat the last; pieces past K repeat the row's last piece (their
+        // groups are not used).
         const int pc = tid & 15, rr = tid >> 4;
-        auto wrow = [&](int j) { const int r = n0 + rr + 16 * j; return Wg + (size_t)(r < N ? r : N - 1) * K; };
         auto xcol = [&](int j) {
             const int c = imin(c0 + rr + 16 * j, ncols - 1);
             int xr = c;
@@ -213,8 +176,7 @@ __global__ __launch_bounds__(MF_THREADS) void k_mfma_q8(const int8_t *__restrict
             }
             return X + (size_t)xr * K;
         };
-        const int8_t *wl0 = wrow(0), *wl1 = wrow(imin(1, MF_RT - 1)), *wl2 = wrow(imax(0, MF_RT - 2)),
-                     *wl3 = wrow(MF_RT - 1);
+        const int8_t *wl0 = Wg + (size_t)imin(n0 + rr, N - 1) * K;
         const int8_t *xl0 = xcol(0), *xl1 = xcol(1), *xl2 = xcol(2), *xl3 = xcol(3);
         // the activation scales this thread stages: column tid / 4
         const float *xsl;
@@ -228,13 +190,9 @@ __global__ __launch_bounds__(MF_THREADS) void k_mfma_q8(const int8_t *__restrict
             xsl = Xs + (size_t)xr * nb;
         }
         const int nst = (K + MF_KC - 1) / MF_KC;
-        int4 Aw0, Aw1 = {}, Aw2 = {}, Aw3 = {}, Ax0, Ax1, Ax2, Ax3;
+        int4 Aw0, Ax0, Ax1, Ax2, Ax3;
         float At0, At1;
-        float f[MF_RT][4];
-#pragma unroll
-        for (int i = 0; i < MF_RT; i++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) f[i][v] = 0.0f;
+        float f[4] = {0.0f, 0.0f, 0.0f, 0.0f};
         // one group (K == 32): f holds the exact group sum (|acc| < 2^24) for
         // epi_one_group's association
         const bool one = nb == 1;
@@ -261,16 +219,13 @@ __global__ __launch_bounds__(MF_THREADS) void k_mfma_q8(const int8_t *__restrict
         if (cl < ncols) {
             float *op = out + (size_t)orow * out_stride;
 #pragma unroll
-            for (int i = 0; i < MF_RT; i++) {
-#pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    const int n = n0 + 16 * i + 4 * (lane >> 4) + v;
-                    if (n < N) {
-                        float sum = 0.0f;
-                        if (one) sum = epi_one_group((int)f[i][v], s0, wsg[n]);
-                        else sum += f[i][v] * wsg[n];
-                        op[n] = sum;
-                    }
+            for (int v = 0; v < 4; v++) {
+                const int n = n0 + 4 * (lane >> 4) + v;
+                if (n < N) {
+                    float sum = 0.0f;
+                    if (one) sum = epi_one_group((int)f[v], s0, wsg[n]);
+                    else sum += f[v] * wsg[n];
+                    op[n] = sum;
                 }
             }
         }
@@ -820,11 +775,15 @@ extern "C" int l98k_upload_exp_table_mfma(const float *tab) {
 }
 
 // The tile of k_mfma_q8t's launches: 32 weight rows x 16 token columns for at
-// most 16 columns, 64 x 32 where that still leaves MFT_BIG tiles or more (four
-// rounds of the chip's 512 block places), else 32 x 32.  Measured (us, rows x
-// K at that many columns; 32 x 16 / 32 x 32 / 64 x 32 tiles; before, on tiles
+// most 16 columns, 64 x 32 where that still leaves MFT_BIG tiles or more (by its
+// LDS three blocks to a CU, 768 on the chip), else 32 x 32.  Measured (us, rows
+// x K at that many columns; 32 x 16 / 32 x 32 / 64 x 32 tiles; before, on tiles
 // of 64 x 16 up to 128 columns and 16 x 64 above):
+//     2048 x 1024 at   1:   5.0 /  5.2 /  7.2 (5.9)
 //     4176 x 1024 at  12:   5.5 /  5.6 /  7.8 (6.8)
+//    65536 x 1024 at   8:  14.4 / 15.2 / 16.8 (17.3)
+//   131072 x 2048 at   4:  40.5 / 41.9 / 45.1 (47.1)
+//   131072 x 2048 at  16:  43.0 / 45.5 / 46.6 (48.2)
 //     2048 x 2048 at 128:   8.3 /  8.1 / 11.8 (9.8)
 //     8336 x 2048 at 128:  16.9 / 16.8 / 16.5 (22.1)
 //   131072 x 2048 at 128:   233 /  201 /  174 (254)
