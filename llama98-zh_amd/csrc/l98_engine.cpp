@@ -1809,9 +1809,10 @@ namespace {
 // at V = 65536 0.32 ms alone), into pinned memory it runs at the link's rate (1.3
 // ms and 0.03 ms).  Non-coherent (only copies write it, and the stream is waited
 // for before it is read), and cleared by the device, at the link's rate (60 us
-// for 2.7 MB) while the host goes on: the caller waits for d->st.  (The host's
-// first touch of 2.7 MB takes 1.0 ms of page faults, which it now takes only for
-// the pages it reads.)  A block of 2.7 MB takes 0.35 ms to pin and 5.5 MB 0.6, so
+// for 2.7 MB) while the host goes on: the caller waits for d->st.  (After the
+// arena's allocation: beside it, new device memory took 0.25 ms more to map.  The
+// host's first touch of 2.7 MB takes 1.0 ms of page faults, which it now takes
+// only for the pages it reads.)  A block of 2.7 MB takes 0.35 ms to pin and 5.5 MB 0.6, so
 // a freed session's goes to the next (its stream was waited for); pageable when
 // the host has no memory to pin.
 bool mirrors_alloc(LZRunState *s, DState *d, const LZModelConfig &c) {
@@ -2012,9 +2013,9 @@ int batch_capture_dev(DState *d, LZRunState *s, const int *tokens, int n, int po
         // others' GEMMs, paid while the recurrence was three times as long and
         // the GEMMs had 16-row tiles: the many small launches and the waits
         // between streams now cost what they hide.  511 rows of the 24-layer
-        // model take 7.8 ms on one stream, 6.0 to 10 ms on two or three
-        // depending on which hardware queues a process's streams share; 99
-        // rows 4.1 and 6.0 ms.)
+        // model took 7.8 ms on one stream when the parts went, 6.0 to 10 ms on
+        // two or three depending on which hardware queues a process's streams
+        // share, 99 rows 4.1 and 6.0 ms; 511 rows 5.9 ms since.)
         for (int done = 0; done < n;) {
             const int k = n - done < w->cap ? n - done : w->cap;
             h.pos_scratch = pos0 + done;
