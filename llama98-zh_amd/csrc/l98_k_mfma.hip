@@ -403,8 +403,8 @@ __global__ __launch_bounds__(MF_THREADS) void k_mfma_q8n(const int8_t *__restric
 #undef MFN_STAGE_LOAD
 #undef MFN_STAGE_PUT
 
-// The tiled form, for many columns per weight row: a block of four waves (2
-// x 2) computes 32 RT weight rows x 32 CT token columns, a wave 16 RT x 16 CT
+// The tiled form, for many columns per weight row: a block of WR x WC waves
+// computes 16 RT WR weight rows x 16 CT WC token columns, a wave 16 RT x 16 CT
 // (RT x CT MFMA tiles per group, whose operands are read from LDS RT + CT
 // times).  K goes through LDS in stages of 128 bytes (four groups) in four
 // buffers, loaded by the LDS direct loads (no registers, no store
